@@ -188,7 +188,7 @@ struct Sink {
 
 // Buffers of the batched prompt prefill (per model, grown on demand).
 struct PfBufs {
-    int cap = 0;                 // token rows (multiple of 64) the row buffers hold
+    int cap = 0;                 // token rows (multiple of 128) the row buffers hold
     float* x = nullptr;          // [cap][H] residual after attention / after the layer
     float* x1 = nullptr;         // [cap][H] residual after attention
     void* a = nullptr;           // [2][cap][Kmax] fp16 (Q4_0 weights) or [cap][Kmax] f32: GEMM operand
@@ -318,7 +318,9 @@ int enqueue_persistent(gh_model* m, gh_kv* kv, Sink& sink, int pos);
 // selection of the last of them (position pos0+n-1).
 constexpr int PF_MAX_TOKENS = 512;  // tokens per prefill pass
 constexpr int PF_ATTN_NC = 16;      // attention chunks per token and kv head in the prefill
-int pf_splits(const DMat& w, int Pp, int* kb_per);
+int pf_tile_rows(int fmt, int n);
+int pf_rows_padded(int fmt, int n);
+int pf_splits(const DMat& w, int n, int* kb_per);
 int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool head);
 int launch_q4_dequant(const DMat& w, float* out, hipStream_t s);
 int launch_matvec_plain(const DMat& w, const Plan& p, const float* x, float* part, float* y,

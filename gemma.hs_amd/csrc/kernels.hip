@@ -266,6 +266,16 @@ struct BufView {
     __device__ __forceinline__ u32x2 u2(uint32_t off) const {
         return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, CP));
     }
+    // the same with a wave-uniform byte offset `so` added (a scalar operand); off + so stays in range
+    __device__ __forceinline__ u32x4 u4s(uint32_t off, uint32_t so) const {
+        return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, so, 0));
+    }
+    __device__ __forceinline__ u32x2 u2s(uint32_t off, uint32_t so) const {
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, so, 0));
+    }
+    __device__ __forceinline__ uint16_t h1s(uint32_t off, uint32_t so) const {
+        return __builtin_amdgcn_raw_buffer_load_b16(r, off, so, 0);
+    }
     template <int CP = 0>
     __device__ __forceinline__ float f1(uint32_t off) const {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, CP));
@@ -4187,6 +4197,7 @@ int enqueue_step(gh_model* m, gh_kv* kv, Sink& sink, int pos) {
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 // GEMM operand A, [Pp][K] per part.
 // With Q4_0 weights (split = 1), each token row t is first scaled by a power
@@ -4194,10 +4205,8 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // The row is then stored as two fp16 parts hi + lo.  Per element the error
 // |x - (hi + lo) / scale| is at most 2^-23 |x| + 2^-40 max|x|, which is below
 // f32 rounding.  (q - 8) * part is exact in the MFMA's f32 products.
-// The columns of every 32-column block are permuted to match the weight
-// fragments: lane group g of an MFMA holds columns
-// {4g, 4g+2, 4g+1, 4g+3, 16+4g, 16+4g+2, 16+4g+1, 16+4g+3}, the low and
-// high nibbles of code bytes 4g..4g+3 as q4_f16_pair unpacks them.
+// Columns 4j..4j+3 are stored in the order 0, 2, 1, 3, in which q4_f16x8
+// unpacks the nibbles of a code dword.
 // With f32 weights (split = 0): plain f32, unscaled.
 struct PfA {
     void* p;
@@ -4210,8 +4219,7 @@ struct PfA {
             *(float4*)((float*)p + (size_t)t * K + k) = v;
             return;
         }
-        const int kk = k & 31;
-        const size_t at = (size_t)t * K + (k & ~31) + (kk < 16 ? 2 * kk : 2 * kk - 28);
+        const size_t at = (size_t)t * K + k;
         const float x[4] = {v.x * sc, v.z * sc, v.y * sc, v.w * sc};  // stored order 0, 2, 1, 3
         uint32_t hi[4], lo[4];
 #pragma unroll
@@ -4381,125 +4389,198 @@ __device__ __forceinline__ bool pf_tile(const PfGemm& g, PfTile& t) {
 }
 inline int pf_grid(int X, int Y, int S) { return (X * S + 7) / 8 * 8 * Y; }
 
-// (q - 8) as fp16 for the two nibbles of w at bits [s, s+4) and [s+16, s+20):
-// 1024 + q is 0x6400 | q in fp16, and 1024 + q - 1032 is exact.
-__device__ __forceinline__ uint32_t q4_f16_pair(uint32_t w, int s) {
-    const uint32_t v = ((w >> s) & 0x000F000Fu) | 0x64006400u;
-    const f16x2_t h = __builtin_bit_cast(f16x2_t, v) - f16x2_t{(_Float16)1032.0f, (_Float16)1032.0f};
-    return __builtin_bit_cast(uint32_t, h);
+// (q - 8) as fp16 for 8 nibbles of a row's code dwords w0, w1 (8 code bytes):
+// HI = 0 the low ones, HI = 1 the high ones, in the column order 0, 2, 1, 3,
+// 4, 6, 5, 7.  1024 + q is 0x6400 | q in fp16 and 1024 + 16q is 0x6400 |
+// (q << 4); subtracting 1032, or the fma (1024 + 16q) / 16 - 72, is exact.
+// `bias` holds 0x64006400 in a VGPR (pf_bias), so that mask and bias are one
+// v_and_or_b32 (a VOP3 reads one scalar constant).
+__device__ __forceinline__ uint32_t pf_bias() {
+    uint32_t r;
+    asm("v_mov_b32 %0, 0x64006400" : "=v"(r));
+    return r;
+}
+template <int HI>
+__device__ __forceinline__ f16x8_t q4_f16x8(uint32_t w0, uint32_t w1, uint32_t bias) {
+    auto pair = [&](uint32_t w) {
+        if constexpr (HI) {
+            const f16x2_t h = __builtin_bit_cast(f16x2_t, (w & 0x00F000F0u) | bias);
+            return __builtin_elementwise_fma(h, f16x2_t{(_Float16)0.0625f, (_Float16)0.0625f},
+                                             f16x2_t{(_Float16)-72.0f, (_Float16)-72.0f});
+        } else {
+            const f16x2_t h = __builtin_bit_cast(f16x2_t, (w & 0x000F000Fu) | bias);
+            return h - f16x2_t{(_Float16)1032.0f, (_Float16)1032.0f};
+        }
+    };
+    const f16x2_t a = pair(w0), b = pair(w0 >> 8), c = pair(w1), d = pair(w1 >> 8);
+    return f16x8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
-// The 8 fp16 weights of code dword w (bytes 4g..4g+3 of a row's block), in
-// the order of the A column permutation.
-__device__ __forceinline__ uint4 q4_f16_frag(uint32_t w) {
-    return make_uint4(q4_f16_pair(w, 0), q4_f16_pair(w, 8), q4_f16_pair(w, 4), q4_f16_pair(w, 12));
-}
-
-constexpr int PF_DEPTH = 4;  // column blocks in flight per workgroup
-
-// LDS slot of B-operand lane s (0..63) of a fragment: s ^ 4 * (s / 16).  The
-// 16 lanes of a write phase (4 rows x the 4 k-groups of one code dword's
-// row) and of a read phase (16 lanes of one k-group) then fall on 16
-// different 16-byte bank groups (without it, a row's four k-groups sit
-// 256 bytes apart: the same banks).
-__device__ __forceinline__ int pf_swz(int s) { return s ^ ((s >> 4) << 2); }
-
-// Q4_0 weights on v_mfma_f32_16x16x32_f16.  Workgroup = 64 token rows x
-// 16*NS weight rows (NS = 8: one 128-row tile, NS = 4: half a tile) x one
-// split; wave w owns token rows 16w..16w+15 and all NS row subtiles.
-// Per 32-column block (one MFMA K step):
-//   1. the workgroup unpacks the block's codes of its rows once into LDS as
-//      fp16 fragments, and its scales as f32;
-//   2. each wave runs 2 MFMAs (hi, lo parts of A) per row subtile into a
-//      fresh accumulator, then adds d * that to the running sum.
-// Codes, scales and A fragments are loaded PF_DEPTH blocks ahead.  The LDS
-// fragments are double-buffered, with one barrier per block.
-template <int NS>
-__global__ __launch_bounds__(NT) void k_pf_gemm_q4(PfGemm g) {
-    constexpr int R = 16 * NS;       // weight rows per workgroup
-    constexpr int NI = R * 4 / NT;   // code dwords per thread per block
-    static_assert(NI >= 1 && NI * NT == R * 4, "NS must be 4 or 8");
-    __shared__ __align__(16) uint4 bs[2][NS][64];
-    __shared__ float ss[2][R];
+// Q4_0 weights on v_mfma_f32_16x16x32_f16.  Workgroup = 16*TM*MW token rows x
+// one 128-row weight tile x one split; the 4 waves are MW (tokens) x 4/MW
+// (rows), each with 16*TM tokens x 16*TN rows.  Per 32-column block:
+//   - the workgroup's A goes through LDS, double-buffered, its loads two
+//     blocks ahead in registers; one barrier per block;
+//   - wave w unpacks the codes and scales of rows 32w .. 32w+31 into LDS a
+//     block ahead, once for the MW waves that use them;
+//   - 2 chained MFMAs (lo and hi parts) per 16 x 16 subtile into a fresh
+//     accumulator; d * that is added to the sum behind the next subtiles'
+//     MFMAs.
+// The 128 x 128 tile takes 0.55 us per block and CU, whether one or two
+// workgroups share the CU: per wave 32 MFMAs (512 cycles), 95 VALU
+// instructions (64 of them the scale FMAs) and 20 LDS ones.  Four blocks in
+// flight instead of two, stages of two or four blocks per barrier and
+// v_mfma_f32_32x32x16_f16 measured the same.  Against the 64 x 128 tile it
+// replaced (16 tokens a wave, whose LDS reads took as long as its MFMAs), 512
+// tokens: 1B gate/up 49 -> 43 us, 4B gate/up 135 -> 122, qkv 45 -> 30, down
+// 79 -> 66.
+template <int MW, int TM, int TN>
+__global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
+    constexpr int NW = 4 / MW, MT = 16 * TM * MW;
+    static_assert(16 * TN * NW == TILE_ROWS, "a workgroup covers one weight tile");
+    constexpr int CH = MT / 16 * 2;           // 1 KB chunks of A per block: 16 tokens x 32 columns of one part
+    constexpr int CW = CH >= 4 ? CH / 4 : 1;  // chunks a staging wave takes
+    __shared__ __align__(16) u32x4 as[2][CH][64];
+    __shared__ __align__(16) f16x8_t bs[2][4][2][64];  // [row group of 32][low, high nibbles][row + 32 * (code half)]
+    __shared__ float ds[2][TILE_ROWS];
     PfTile pt;
     if (!pf_tile(g, pt)) return;  // uniform per workgroup
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int tile = pt.x / (8 / NS), r0 = (pt.x % (8 / NS)) * R;
-    const int t0 = pt.y * 64 + 16 * wave;
+    const int wave = wave_id(), lane = threadIdx.x & 63;
+    const int wm = wave / NW, wn = wave % NW;
+    const int t0 = pt.y * MT;
     const int kb0 = pt.z * g.kb_per, nk = min(g.w.nblk, kb0 + g.kb_per) - kb0;
     const int K = g.a.K;
-    const size_t pstride = (size_t)g.a.Pp * K;
-    const uint16_t* abase = (const uint16_t*)g.a.p + (size_t)(t0 + (lane & 15)) * K + 8 * (lane >> 4);
-    const uint32_t* codes = (const uint32_t*)g.w.codes + ((size_t)tile * g.w.nblk + kb0) * TILE_ROWS * 4 + r0 * 4;
-    const uint16_t* scales = g.w.scales + ((size_t)tile * g.w.nblk + kb0) * TILE_ROWS + r0;
-    // code dword item = tid + NT*q of the block's R x 4 -> (row = item >> 2,
-    // g = item & 3) -> LDS fragment (subtile row >> 4, lane (row & 15) + 16 g)
-    uint4* frag[NI];
+    const int m16 = lane & 15, kg = lane >> 4;  // MFMA operand row, columns 8 kg .. 8 kg + 7 of the block
+    // A chunk: row r of 16 at r * 64 bytes, its 16-byte piece p at slot p ^
+    // f(r), so that an operand read (one piece of rows 0 .. 15 per cycle)
+    // falls on 16 different bank groups
+    auto f = [](int r) { return (r >> 2) & 3; };
+    const BufView A((const uint16_t*)g.a.p + (size_t)t0 * K, ((size_t)g.a.Pp * K + (size_t)MT * K) * 2);
+    uint32_t ao[CW];
 #pragma unroll
-    for (int q = 0; q < NI; ++q) {
-        const int item = tid + NT * q, row = item >> 2;
-        frag[q] = &bs[0][row >> 4][pf_swz((row & 15) + 16 * (item & 3))];
+    for (int q = 0; q < CW; ++q) {
+        const int c = wave * CW + q, part = c / (MT / 16), r = lane >> 2;
+        ao[q] = 2u * ((uint32_t)part * (uint32_t)g.a.Pp * K + (uint32_t)(c % (MT / 16) * 16 + r) * K + 8u * ((lane & 3) ^ f(r)));
     }
-    uint32_t rb[PF_DEPTH][NI];
-    uint16_t rs[PF_DEPTH];
-    uint4 ra0[PF_DEPTH], ra1[PF_DEPTH];
-    // Block i's loads into ring slot j.  Every call issues the same loads
-    // (indices clamped into range, no branches), so the wait counts stay
-    // static and the PF_DEPTH blocks in flight are not drained early.
+    const size_t we = (size_t)pt.x * g.w.nblk * TILE_ROWS;  // the tile's first (row, block)
+    const BufView C((const uint8_t*)g.w.codes + we * 16, (size_t)g.w.nblk * TILE_ROWS * 16);
+    const BufView S(g.w.scales + we, (size_t)g.w.nblk * TILE_ROWS * 2);
+    const uint32_t urow = (uint32_t)(32 * wave + (lane & 31));  // the row this lane unpacks
+    u32x4 ra[2][CW];
+    u32x2 rb[2];
+    uint16_t rs[2];
+    // Loads of block i into ring slot j.  Past the split's last block they
+    // read that block again and its scales count as zeros, so that a split
+    // runs an even number of blocks with no branch between the loads and
+    // their use (the compiler would sink them to it).
     auto load = [&](int j, int i) {
-        const int ic = min(i, nk - 1);
-        const uint32_t* cb = codes + (size_t)ic * TILE_ROWS * 4;
+        const uint32_t kb = (uint32_t)(kb0 + min(i, nk - 1));
+        rb[j] = C.u2s(urow * 16 + 8 * (lane >> 5), kb * TILE_ROWS * 16);
+        rs[j] = S.h1s(urow * 2, kb * TILE_ROWS * 2);
 #pragma unroll
-        for (int q = 0; q < NI; ++q) rb[j][q] = cb[tid + NT * q];
-        rs[j] = scales[(size_t)ic * TILE_ROWS + min(tid, R - 1)];
-        const uint16_t* ap = abase + (size_t)(kb0 + ic) * 32;
-        ra0[j] = *(const uint4*)ap;
-        ra1[j] = *(const uint4*)(ap + pstride);
+        for (int q = 0; q < CW; ++q)
+            if (CH >= 4 || wave < CH) ra[j][q] = A.u4s(ao[q], 64u * kb);
     };
-    f32x4_t acc[NS];
+    const uint32_t bias = pf_bias();
+    // block i from slot j into LDS buffer j
+    auto unpack = [&](int j, int i) {
+        bs[j][wave][0][lane] = q4_f16x8<0>(rb[j].x, rb[j].y, bias);
+        bs[j][wave][1][lane] = q4_f16x8<1>(rb[j].x, rb[j].y, bias);
+        ds[j][urow] = i < nk ? h2f(rs[j]) : 0.0f;  // both code halves' lanes write the same value
+    };
+    auto store_a = [&](int j) {
 #pragma unroll
-    for (int n = 0; n < NS; ++n) acc[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int q = 0; q < CW; ++q)
+            if (CH >= 4 || wave < CH) as[j][wave * CW + q][lane] = ra[j][q];
+    };
+    f32x4_t acc[TM][TN];
 #pragma unroll
-    for (int j = 0; j < PF_DEPTH; ++j) load(j, j);
-    for (int base = 0; base < nk; base += PF_DEPTH) {
+    for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int j = 0; j < PF_DEPTH; ++j) {
+        for (int n = 0; n < TN; ++n) acc[m][n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    load(0, 0);
+    load(1, 1);
+    unpack(0, 0);
+    store_a(0);
+    __syncthreads();
+    // products of the last token subtiles, added while the next ones' MFMAs run
+    f32x4_t cp[TN];
+    float dp[TN];
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+        cp[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        dp[n] = 0.0f;
+    }
+    for (int base = 0; base < nk; base += 2) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
             const int i = base + j;
-            if (i >= nk) break;
-            const int buf = j & 1;  // == i & 1: PF_DEPTH is even
+            auto read_a = [&](int m, int p) {
+                return __builtin_bit_cast(f16x8_t, as[j][p * (MT / 16) + wm * TM + m][m16 * 4 + (kg ^ f(m16))]);
+            };
+            f16x8_t b[TN], a[2];
+            float d[TN];
+            a[1] = read_a(0, 1);
+            a[0] = read_a(0, 0);
 #pragma unroll
-            for (int q = 0; q < NI; ++q) frag[q][buf * NS * 64] = q4_f16_frag(rb[j][q]);
-            if (tid < R) ss[buf][tid] = h2f(rs[j]);
-            const f16x8_t a0 = __builtin_bit_cast(f16x8_t, ra0[j]);
-            const f16x8_t a1 = __builtin_bit_cast(f16x8_t, ra1[j]);
-            __syncthreads();
-            load(j, i + PF_DEPTH);
-#pragma unroll
-            for (int n = 0; n < NS; ++n) {
-                const f16x8_t b = __builtin_bit_cast(f16x8_t, bs[buf][n][pf_swz(lane)]);
-                const float d = ss[buf][16 * n + (lane & 15)];
-                f32x4_t c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b, c, 0, 0, 0);
-                acc[n] += d * c;
+            for (int n = 0; n < TN; ++n) {
+                const int r = 16 * (TN * wn + n) + m16;
+                b[n] = bs[j][r >> 5][kg >> 1][(r & 31) + 32 * (kg & 1)];
+                d[n] = ds[j][r];
             }
+            load(j, i + 2);
+#pragma unroll
+            for (int m = 0; m < TM; ++m) {
+                f16x8_t an[2] = {a[0], a[1]};
+                if (m + 1 < TM) {
+                    an[1] = read_a(m + 1, 1);
+                    an[0] = read_a(m + 1, 0);
+                }
+                f32x4_t c[TN];
+#pragma unroll
+                for (int n = 0; n < TN; ++n)
+                    c[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[1], b[n], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                for (int n = 0; n < TN; ++n) c[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[n], c[n], 0, 0, 0);
+#pragma unroll
+                for (int n = 0; n < TN; ++n) {
+                    acc[(m + TM - 1) % TM][n] += dp[n] * cp[n];
+                    cp[n] = c[n];
+                    dp[n] = d[n];
+                }
+                if (m == TM / 2) unpack(j ^ 1, i + 1);
+                if (m == TM - 1) store_a(j ^ 1);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the next operands' reads first
+#pragma unroll
+                for (int t = 0; t < 2 * TN; ++t) {  // then VALU work between the MFMAs
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                a[0] = an[0];
+                a[1] = an[1];
+            }
+            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // lane holds token rows 4*(lane>>4) .. +3 of the wave's 16, weight row
-    // r0 + 16 n + (lane & 15) of the tile
-    const int tr = t0 + 4 * (lane >> 4);
-    float inv[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) inv[r] = g.a.inv_scale[tr + r];
-    float* o = g.out + ((size_t)pt.z * g.a.Pp + tr) * g.ldo + (size_t)tile * TILE_ROWS + r0 + (lane & 15);
+    for (int n = 0; n < TN; ++n) acc[TM - 1][n] += dp[n] * cp[n];
+    // lane holds weight row 16 n + m16 of the wave's, tokens 4 kg .. 4 kg + 3 of each 16
 #pragma unroll
-    for (int n = 0; n < NS; ++n)
+    for (int m = 0; m < TM; ++m) {
+        const int tw = t0 + 16 * (wm * TM + m) + 4 * kg;
+        const float4 inv = *(const float4*)(g.a.inv_scale + tw);
+        float* o = g.out + ((size_t)pt.z * g.a.Pp + tw) * g.ldo + (size_t)pt.x * TILE_ROWS + 16 * TN * wn + m16;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[(size_t)r * g.ldo + 16 * n] = acc[n][r] * inv[r];
+        for (int n = 0; n < TN; ++n) {
+            o[16 * n] = acc[m][n][0] * inv.x;
+            o[(size_t)g.ldo + 16 * n] = acc[m][n][1] * inv.y;
+            o[2 * (size_t)g.ldo + 16 * n] = acc[m][n][2] * inv.z;
+            o[3 * (size_t)g.ldo + 16 * n] = acc[m][n][3] * inv.w;
+        }
+    }
 }
-
-// Row-subtiles per workgroup of a Q4_0 prefill GEMM: whole tiles, unless
-// even 8 splits leave fewer than 512 workgroups; then half tiles.
-static int pf_ns(const DMat& w, int Pp) { return w.tiles * (Pp / 64) * 8 >= 512 ? 8 : 4; }
 
 // f32 weights on v_mfma_f32_16x16x4_f32: one 4-column block per MFMA.
 __global__ __launch_bounds__(NT) void k_pf_gemm_f32(PfGemm g) {
@@ -4857,19 +4938,45 @@ __global__ __launch_bounds__(NT) void k_pf_geglu(const float* part, int ld, int 
     for (int k = 4 * threadIdx.x; k < F; k += 4 * NT) a.put4(t, k, *(const float4*)&rowbuf[k], sc);
 }
 
-// Split count of a prefill GEMM over Pp token rows, at most 8: enough for
-// two workgroups per CU where the columns are many (K >= 4096: the FFN's
-// down projection, whose workgroups' latency chain bounds it), one per CU
-// otherwise (QKV, O: there the next kernel's reads of the partials cost
-// more than the extra workgroups save).  Measured on MI355X, 512-token
-// prefill: QKV 426 -> 355 us and O 302 -> 267 us at one workgroup per CU;
-// down 831 -> 1048 us, so it keeps two.
-int pf_splits(const DMat& w, int Pp, int* kb_per) {
-    const int wgs = (w.fmt == FMT_Q4 ? w.tiles * (8 / pf_ns(w, Pp)) : 2 * w.tiles) * (Pp / 64);
-    const int target = w.cols >= 4096 ? 512 : 256;
-    int S = std::max(1, std::min(8, (target + wgs - 1) / wgs));
-    S = std::min(S, w.nblk);
-    const int per = (w.nblk + S - 1) / S;
+// Token rows of one GEMM workgroup for a pass of n tokens, and the pass's rows
+// rounded up to whole workgroups.  Q4_0: the smallest tile that holds a short
+// pass (the block time falls with it, see below), else 128.
+int pf_tile_rows(int fmt, int n) { return fmt != FMT_Q4 ? 64 : n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : 128; }
+int pf_rows_padded(int fmt, int n) {
+    const int mt = pf_tile_rows(fmt, n);
+    return (n + mt - 1) / mt * mt;
+}
+
+// Split count of a prefill GEMM over a pass of n tokens, at most 8.  Q4_0:
+// the S whose estimate is lowest of
+//   rounds of workgroups over the CUs x blocks per split x block time
+//   + the S partials' way out and back in (4 B per row and token each)
+// with what MI355X measured: 0.55 / 0.38 / 0.30 / 0.28 us per block at 128 /
+// 64 / 32 / 16 token rows, 0.58 us per MB of partials.  Over sweeps of S at
+// 16 .. 1907 tokens of the 1B and 4B shapes it picks the best S or one whose
+// GEMM plus consumer is within 3 us of it, but for 1024-token 1B down (3
+// splits, 62 us with its consumer; 6 take 55).  f32: two workgroups per CU
+// where the columns are many (K >= 4096, the down projection), else one.
+int pf_splits(const DMat& w, int n, int* kb_per) {
+    const int mt = pf_tile_rows(w.fmt, n), Pp = pf_rows_padded(w.fmt, n);
+    const int wgs = (w.fmt == FMT_Q4 ? w.tiles : 2 * w.tiles) * (Pp / mt);
+    int S = std::max(1, std::min(8, ((w.cols >= 4096 ? 512 : 256) + wgs - 1) / wgs));
+    auto blocks = [&](int splits) {
+        const int per = (w.nblk + splits - 1) / splits;
+        return w.fmt == FMT_Q4 ? (per + 1) & ~1 : per;  // the Q4_0 kernel runs pairs of blocks
+    };
+    if (w.fmt == FMT_Q4) {
+        const double tb = mt == 128 ? 0.55 : mt == 64 ? 0.38 : mt == 32 ? 0.30 : 0.28;
+        double best = 0.0;
+        for (int c = 1; c <= std::min(8, w.nblk); ++c) {
+            const double t = (wgs * c + 255) / 256 * blocks(c) * tb + 0.58e-6 * 4.0 * c * Pp * w.tiles * TILE_ROWS;
+            if (c == 1 || t < best) {
+                best = t;
+                S = c;
+            }
+        }
+    }
+    const int per = blocks(std::min(S, w.nblk));
     if (kb_per) *kb_per = per;
     return (w.nblk + per - 1) / per;
 }
@@ -4882,7 +4989,7 @@ int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool he
     const gh_config& c = m->cfg;
     const PfBufs& B = m->pf;
     const int H = c.hidden, hd = c.head_dim, nkv = c.n_kv_heads, G = c.n_heads / nkv, F = c.ffn;
-    const int Pp = (n + 63) / 64 * 64;
+    const int Pp = pf_rows_padded(m->fmt, n), mt = pf_tile_rows(m->fmt, n);
     if (n <= 0 || Pp > B.cap) return set_error(GH_ERR_INVALID, "internal: prefill of %d rows, buffers hold %d", n, B.cap);
     const int zc = (c.flags & GH_FLAG_ZERO_CENTERED) ? 1 : 0;
     const float eps = c.rms_eps;
@@ -4895,16 +5002,19 @@ int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool he
     // GEMM of operand A (K columns) with w into the partials; returns S
     auto gemm = [&](const char* name, const DMat& w, int* S_out) -> int {
         int per = 0;
-        const int S = pf_splits(w, Pp, &per);
+        const int S = pf_splits(w, n, &per);
         if ((size_t)S * Pp * w.tiles * TILE_ROWS > B.part_floats)
             return set_error(GH_ERR_INVALID, "internal: prefill partials too small");
         *S_out = S;
-        const int ns = w.fmt == FMT_Q4 ? pf_ns(w, Pp) : 4;  // f32: 64-row groups
-        PfGemm g{A(w.cols), w, per, B.part, w.tiles * TILE_ROWS, w.tiles * (8 / ns), Pp / 64, S};
+        // Q4_0: whole tiles a workgroup; f32: 64-row groups
+        PfGemm g{A(w.cols), w, per, B.part, w.tiles * TILE_ROWS, w.fmt == FMT_Q4 ? w.tiles : 2 * w.tiles, Pp / mt, S};
         const dim3 grid(pf_grid(g.X, g.Y, g.S));
+        auto q4 = [&](auto fn) { return sink_launch(sink, name, pf_gemm_bytes(w, n), fn, grid, dim3(NT), 0, g); };
         if (w.fmt == FMT_Q4)
-            return ns == 8 ? sink_launch(sink, name, pf_gemm_bytes(w, n), k_pf_gemm_q4<8>, grid, dim3(NT), 0, g)
-                           : sink_launch(sink, name, pf_gemm_bytes(w, n), k_pf_gemm_q4<4>, grid, dim3(NT), 0, g);
+            return mt == 128  ? q4(k_pf_gemm_q4<2, 4, 4>)
+                   : mt == 64 ? q4(k_pf_gemm_q4<1, 4, 2>)
+                   : mt == 32 ? q4(k_pf_gemm_q4<1, 2, 2>)
+                              : q4(k_pf_gemm_q4<1, 1, 2>);
         return sink_launch(sink, name, pf_gemm_bytes(w, n), k_pf_gemm_f32, grid, dim3(NT), 0, g);
     };
     auto rows = [&](const char* name, PfRows r, int n_rows) {

@@ -389,10 +389,10 @@ void free_prefill(gh_model* m) {
     B = PfBufs{};
 }
 
-// Prefill buffers for passes of up to n tokens (rows rounded up to 64).
+// Prefill buffers for passes of up to n tokens (rows rounded up to 128).
 int prefill_reserve(gh_model* m, int n) {
     const gh_config& c = m->cfg;
-    const int cap = (n + 63) / 64 * 64;
+    const int cap = (n + 127) / 128 * 128;
     if (cap > PF_MAX_TOKENS) return set_error(GH_ERR_INVALID, "internal: prefill pass of %d tokens", n);
     if (m->pf.cap >= cap) return GH_OK;
     GH_HIP(hipStreamSynchronize(m->ctx->stream));
@@ -402,8 +402,8 @@ int prefill_reserve(gh_model* m, int n) {
     const size_t kmax = std::max({(size_t)H, (size_t)nq * hd, (size_t)c.ffn});
     size_t part = 0;
     for (const DMat* w : {&L.qkv, &L.o, &L.gu, &L.down})
-        for (int pp = 64; pp <= cap; pp += 64)
-            part = std::max(part, (size_t)pf_splits(*w, pp, nullptr) * pp * w->tiles * TILE_ROWS);
+        for (int k = 16; k <= cap; k += 16)
+            part = std::max(part, (size_t)pf_splits(*w, k, nullptr) * pf_rows_padded(w->fmt, k) * w->tiles * TILE_ROWS);
     PfBufs& B = m->pf;
     auto get = [&](void** p, size_t bytes) -> int {
         hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));

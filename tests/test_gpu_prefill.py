@@ -173,6 +173,28 @@ def test_prefill_matrix_core_attention_groups_ragged_windows(ctx, nq, nkv):
     np.testing.assert_array_equal(gh.generate(m, kv_a, [na], 5), gh.generate(m, kv_b, [nb], 5))
 
 
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 32, 33, 64, 65, 128, 129, 257])
+def test_prefill_gemm_tile_edges(ctx, n):
+    """Q4_0 prefill GEMM at the edges of its token tiles (16, 32, 64, 128
+    rows), with odd column block counts (hidden 288: 9 blocks, ffn 352: 11)
+    and a ragged last weight tile: the last token's layers and logits against
+    the decode step fed token by token (other kernels, other sums; both are
+    within ACT_TOL / 2 of the oracle elsewhere, so ACT_TOL bounds their
+    difference)."""
+    cfg = _mini4b(gh.MODE_GEMMA3, window=40, layers=2)
+    cfg.hidden, cfg.ffn, cfg.max_seq = 288, 352, 272
+    m = _gpu_model(ctx, cfg, 31, True)
+    toks = gh.synth_tokens(13, "tile", n, cfg.vocab)
+    kv_a, kv_b = gh.KVCache(m, 272), gh.KVCache(m, 272)
+    la, ya, na = gh.prefill(m, kv_a, toks, want_layers=True)
+    for t in toks[:-1]:
+        gh.runGemmaInferenceCached(m, int(t), kv_b, want_logits=False)
+    lb, _, yb, nb = gh.runGemmaInferenceCachedWithLayer0(m, int(toks[-1]), kv_b)
+    for l in range(cfg.n_layers):
+        assert rel_err(ya[l], yb[l]) < ACT_TOL, l
+    assert rel_err(la, lb) < ACT_TOL and na == nb
+
+
 def test_prefill_single_token_equals_step(ctx):
     """A prefill of one token is the decode step of that token."""
     cfg = _mini4b(gh.MODE_GEMMA3, layers=2)
