@@ -316,7 +316,12 @@ int enqueue_persistent(gh_model* m, gh_kv* kv, Sink& sink, int pos);
 // kernels.hip: batched prefill of n tokens (ids in m->pf.tok) at positions
 // pos0 .. pos0+n-1; with `head`, also the final norm, LM head and next-token
 // selection of the last of them (position pos0+n-1).
-constexpr int PF_MAX_TOKENS = 512;  // tokens per prefill pass
+// Tokens per prefill pass.  Longer passes give the GEMMs more workgroups per
+// launch and the per-token kernels more rows per launch: 1907 tokens of the 1B
+// shape 17.6 ms in passes of 512, 11.5 ms in one; 1024 of the 4B shape 8.67 ->
+// 7.90 ms (the largest buffers, 1B at 2048 tokens: 113 MB of gate/up partials,
+// 135 MB of attention states).
+constexpr int PF_MAX_TOKENS = 2048;
 constexpr int PF_ATTN_NC = 16;      // attention chunks per token and kv head in the prefill
 int pf_tile_rows(int fmt, int n);
 int pf_rows_padded(int fmt, int n);

@@ -4960,7 +4960,9 @@ int pf_rows_padded(int fmt, int n) {
 int pf_splits(const DMat& w, int n, int* kb_per) {
     const int mt = pf_tile_rows(w.fmt, n), Pp = pf_rows_padded(w.fmt, n);
     const int wgs = (w.fmt == FMT_Q4 ? w.tiles : 2 * w.tiles) * (Pp / mt);
-    int S = std::max(1, std::min(8, ((w.cols >= 4096 ? 512 : 256) + wgs - 1) / wgs));
+    // the consumers read all partials through one buffer view (below 2 GiB)
+    const int most = (int)std::max<size_t>(1, std::min<size_t>(8, 0x7fffffffu / ((size_t)4 * Pp * w.tiles * TILE_ROWS)));
+    int S = std::max(1, std::min(most, ((w.cols >= 4096 ? 512 : 256) + wgs - 1) / wgs));
     auto blocks = [&](int splits) {
         const int per = (w.nblk + splits - 1) / splits;
         return w.fmt == FMT_Q4 ? (per + 1) & ~1 : per;  // the Q4_0 kernel runs pairs of blocks
@@ -4968,7 +4970,7 @@ int pf_splits(const DMat& w, int n, int* kb_per) {
     if (w.fmt == FMT_Q4) {
         const double tb = mt == 128 ? 0.55 : mt == 64 ? 0.38 : mt == 32 ? 0.30 : 0.28;
         double best = 0.0;
-        for (int c = 1; c <= std::min(8, w.nblk); ++c) {
+        for (int c = 1; c <= std::min(most, w.nblk); ++c) {
             const double t = (wgs * c + 255) / 256 * blocks(c) * tb + 0.58e-6 * 4.0 * c * Pp * w.tiles * TILE_ROWS;
             if (c == 1 || t < best) {
                 best = t;

@@ -149,6 +149,21 @@ def test_prefill_passes_chunks_and_ragged_sizes(ctx):
     np.testing.assert_array_equal(gb, gc)
 
 
+def test_prefill_longer_than_a_pass(ctx):
+    """2100 tokens: one call (passes of 2048 + 52 rows) against the same
+    tokens as prefills of 1000 and 1100, on the f32 tiny model."""
+    cfg = gh.preset("tiny")
+    cfg.max_seq = 2304
+    m = _gpu_model(ctx, cfg, 7, False)
+    toks = gh.synth_tokens(14, "pass", 2100, cfg.vocab)
+    kv_a, kv_b = gh.KVCache(m, 2304), gh.KVCache(m, 2304)
+    la, _, na = gh.prefill(m, kv_a, toks)
+    gh.prefill(m, kv_b, toks[:1000])
+    lb, _, nb = gh.prefill(m, kv_b, toks[1000:])
+    assert len(kv_a) == len(kv_b) == 2100
+    assert rel_err(la, lb) < ACT_TOL and na == nb
+
+
 @pytest.mark.parametrize("nq,nkv", [(4, 4), (8, 1)])
 def test_prefill_matrix_core_attention_groups_ragged_windows(ctx, nq, nkv):
     """head_dim 256 with GQA groups 1 and 8 (the 2 and 4 of the other tests
