@@ -4582,33 +4582,74 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
     }
 }
 
-// f32 weights on v_mfma_f32_16x16x4_f32: one 4-column block per MFMA.
-__global__ __launch_bounds__(NT) void k_pf_gemm_f32(PfGemm g) {
+// f32 weights on v_mfma_f32_16x16x4_f32.  Workgroup = 16*TM token rows x one
+// 128-row weight tile x one split; wave w takes the tile's rows 32w .. 32w+31
+// for all the tokens.  A step is 16 columns: lane (i, q) = (lane % 16, lane /
+// 16) loads columns 4q .. 4q+3 of its A and W rows as one float4 each, and
+// MFMA e of the step multiplies element e of both (the sum runs over every
+// column once, in that order).  At 64 x 32 per wave six loads feed 32 MFMAs
+// of 32 cycles, so operands come straight from L1/L2, PF_F32_DEPTH steps
+// ahead, with no LDS and no barrier.  Each PF_F32_DEPTH steps are summed from
+// zero and then added to the running sum, which keeps the rounding error
+// below that of one chain over all the columns.  1B shape, 300 tokens: gate/up
+// 709 -> 117 us (82 TFLOP/s; the f32 matrix peak this card reaches is 138), down
+// 424 -> 72; the kernel before it waited on one load per MFMA.
+constexpr int PF_F32_DEPTH = 4;
+template <int TM>
+__global__ __launch_bounds__(NT, 2) void k_pf_gemm_f32(PfGemm g) {
+    constexpr int TN = 2, MT = 16 * TM, D = PF_F32_DEPTH;
     PfTile pt;
     if (!pf_tile(g, pt)) return;  // uniform per workgroup
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int tile = pt.x >> 1;
-    const int lr = (pt.x & 1) * 64 + wave * 16 + (lane & 15);
-    const int t0 = pt.y * 64;
-    const int kb0 = pt.z * g.kb_per, kb1 = min(g.w.nblk, kb0 + g.kb_per);
-    const int kq = lane >> 4;
-    const int K = g.a.K;
-    const float* ab = (const float*)g.a.p + (size_t)(t0 + (lane & 15)) * K + kq;
-    const float* wc = (const float*)g.w.codes;
-    f32x4_t acc[4];
+    const int wave = wave_id(), lane = threadIdx.x & 63, i16 = lane & 15, q = lane >> 4;
+    const int t0 = pt.y * MT, K = g.a.K;
+    const int kb0 = pt.z * g.kb_per, ns = (min(g.w.nblk, kb0 + g.kb_per) - kb0) >> 2;  // steps (nblk % 8 == 0)
+    const BufView A((const float*)g.a.p + (size_t)t0 * K + 4 * kb0, ((size_t)MT * K - 4 * kb0) * 4);
+    const BufView W((const float4*)g.w.codes + ((size_t)pt.x * g.w.nblk + kb0) * TILE_ROWS, (size_t)ns * 4 * TILE_ROWS * 16);
+    f32x4_t ra[D][TM], rb[D][TN];
+    // step s into ring slot j; past the split's end A reads its last step again and W zeros
+    auto load = [&](int j, int s) {
+        const uint32_t wo = (uint32_t)(q * TILE_ROWS + 32 * wave + i16) * 16u + (uint32_t)s * (4 * TILE_ROWS * 16);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int kb = kb0; kb < kb1; ++kb) {
-        const float bw = wc[(((size_t)tile * g.w.nblk + kb) * TILE_ROWS + lr) * 4 + kq];
+        for (int n = 0; n < TN; ++n) rb[j][n] = __builtin_bit_cast(f32x4_t, W.u4(s < ns ? wo + 256u * n : OOB));
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
-            acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(ab[(size_t)(16 * m) * K + 4 * kb], bw, acc[m], 0, 0, 0);
+        for (int m = 0; m < TM; ++m)
+            ra[j][m] = __builtin_bit_cast(f32x4_t, A.u4s(4u * (uint32_t)((16 * m + i16) * K + 4 * q), 64u * (uint32_t)min(s, ns - 1)));
+    };
+    f32x4_t acc[TM][TN];
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int n = 0; n < TN; ++n) acc[m][n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < D; ++j) load(j, j);
+    for (int base = 0; base < ns; base += D) {
+        f32x4_t c[TM][TN];
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int m = 0; m < TM; ++m)
+#pragma unroll
+                    for (int n = 0; n < TN; ++n)
+                        c[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            ra[j][m][e], rb[j][n][e], j + e ? c[m][n] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+            load(j, base + D + j);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int n = 0; n < TN; ++n) acc[m][n] += c[m][n];
     }
-    float* o = g.out + ((size_t)pt.z * g.a.Pp + t0 + 4 * kq) * g.ldo + (size_t)tile * TILE_ROWS + lr;
+    // lane holds weight row 32 wave + 16 n + i16 of the tile, tokens 4 q .. 4 q + 3 of each 16
+    float* o = g.out + ((size_t)pt.z * g.a.Pp + t0 + 4 * q) * g.ldo + (size_t)pt.x * TILE_ROWS + 32 * wave + i16;
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[(size_t)(16 * m + r) * g.ldo] = acc[m][r];
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[(size_t)(16 * m + r) * g.ldo + 16 * n] = acc[m][n][r];
 }
 
 // q/k/v of token t, kv head g: sum of the QKV split partials, QK-norm
@@ -4939,46 +4980,44 @@ __global__ __launch_bounds__(NT) void k_pf_geglu(const float* part, int ld, int 
 }
 
 // Token rows of one GEMM workgroup for a pass of n tokens, and the pass's rows
-// rounded up to whole workgroups.  Q4_0: the smallest tile that holds a short
-// pass (the block time falls with it, see below), else 128.
-int pf_tile_rows(int fmt, int n) { return fmt != FMT_Q4 ? 64 : n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : 128; }
+// rounded up to whole workgroups: the smallest tile that holds a short pass
+// (the block time falls with it, see below), else 128 (f32: 64).
+int pf_tile_rows(int fmt, int n) { return n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 || fmt != FMT_Q4 ? 64 : 128; }
 int pf_rows_padded(int fmt, int n) {
     const int mt = pf_tile_rows(fmt, n);
     return (n + mt - 1) / mt * mt;
 }
 
-// Split count of a prefill GEMM over a pass of n tokens, at most 8.  Q4_0:
-// the S whose estimate is lowest of
-//   rounds of workgroups over the CUs x blocks per split x block time
+// Split count of a prefill GEMM over a pass of n tokens, at most 8: the S
+// whose estimate is lowest of
+//   rounds of workgroups over the CUs x steps per split x step time
 //   + the S partials' way out and back in (4 B per row and token each)
-// with what MI355X measured: 0.55 / 0.38 / 0.30 / 0.28 us per block at 128 /
-// 64 / 32 / 16 token rows, 0.58 us per MB of partials.  Over sweeps of S at
-// 16 .. 1907 tokens of the 1B and 4B shapes it picks the best S or one whose
-// GEMM plus consumer is within 3 us of it, but for 1024-token 1B down (3
-// splits, 62 us with its consumer; 6 take 55).  f32: two workgroups per CU
-// where the columns are many (K >= 4096, the down projection), else one.
+// with what MI355X measured: 0.55 / 0.38 / 0.30 / 0.28 us per 32-column Q4_0
+// block at 128 / 64 / 32 / 16 token rows, 0.55 / 0.33 / 0.21 us per
+// 16-column f32 step at 64 / 32 / 16, 0.58 us per MB of partials.  Over
+// sweeps of S at 16 .. 1907 tokens of the 1B and 4B shapes it picks the best
+// S or one whose GEMM plus consumer is within 3 us of it, but for 1024-token
+// 1B down (3 splits, 62 us with its consumer; 6 take 55).
 int pf_splits(const DMat& w, int n, int* kb_per) {
-    const int mt = pf_tile_rows(w.fmt, n), Pp = pf_rows_padded(w.fmt, n);
-    const int wgs = (w.fmt == FMT_Q4 ? w.tiles : 2 * w.tiles) * (Pp / mt);
+    const int mt = pf_tile_rows(w.fmt, n), Pp = pf_rows_padded(w.fmt, n), wgs = w.tiles * (Pp / mt);
+    const bool q4 = w.fmt == FMT_Q4;
+    // Q4_0: the kernel runs pairs of blocks; f32: steps of 4 blocks, whole rounds of its ring
+    const int unit = q4 ? 2 : 4 * PF_F32_DEPTH;
+    auto blocks = [&](int splits) { return ((w.nblk + splits - 1) / splits + unit - 1) / unit * unit; };
+    const double tb = q4 ? (mt == 128 ? 0.55 : mt == 64 ? 0.38 : mt == 32 ? 0.30 : 0.28)
+                         : (mt == 64 ? 0.55 : mt == 32 ? 0.33 : 0.21) / 4;
     // the consumers read all partials through one buffer view (below 2 GiB)
     const int most = (int)std::max<size_t>(1, std::min<size_t>(8, 0x7fffffffu / ((size_t)4 * Pp * w.tiles * TILE_ROWS)));
-    int S = std::max(1, std::min(most, ((w.cols >= 4096 ? 512 : 256) + wgs - 1) / wgs));
-    auto blocks = [&](int splits) {
-        const int per = (w.nblk + splits - 1) / splits;
-        return w.fmt == FMT_Q4 ? (per + 1) & ~1 : per;  // the Q4_0 kernel runs pairs of blocks
-    };
-    if (w.fmt == FMT_Q4) {
-        const double tb = mt == 128 ? 0.55 : mt == 64 ? 0.38 : mt == 32 ? 0.30 : 0.28;
-        double best = 0.0;
-        for (int c = 1; c <= std::min(most, w.nblk); ++c) {
-            const double t = (wgs * c + 255) / 256 * blocks(c) * tb + 0.58e-6 * 4.0 * c * Pp * w.tiles * TILE_ROWS;
-            if (c == 1 || t < best) {
-                best = t;
-                S = c;
-            }
+    int S = 1;
+    double best = 0.0;
+    for (int c = 1; c <= std::min(most, w.nblk); ++c) {
+        const double t = (wgs * c + 255) / 256 * blocks(c) * tb + 0.58e-6 * 4.0 * c * Pp * w.tiles * TILE_ROWS;
+        if (c == 1 || t < best) {
+            best = t;
+            S = c;
         }
     }
-    const int per = blocks(std::min(S, w.nblk));
+    const int per = blocks(S);
     if (kb_per) *kb_per = per;
     return (w.nblk + per - 1) / per;
 }
@@ -5008,16 +5047,16 @@ int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool he
         if ((size_t)S * Pp * w.tiles * TILE_ROWS > B.part_floats)
             return set_error(GH_ERR_INVALID, "internal: prefill partials too small");
         *S_out = S;
-        // Q4_0: whole tiles a workgroup; f32: 64-row groups
-        PfGemm g{A(w.cols), w, per, B.part, w.tiles * TILE_ROWS, w.fmt == FMT_Q4 ? w.tiles : 2 * w.tiles, Pp / mt, S};
-        const dim3 grid(pf_grid(g.X, g.Y, g.S));
-        auto q4 = [&](auto fn) { return sink_launch(sink, name, pf_gemm_bytes(w, n), fn, grid, dim3(NT), 0, g); };
+        const PfGemm g{A(w.cols), w, per, B.part, w.tiles * TILE_ROWS, w.tiles, Pp / mt, S};
+        auto go = [&](auto fn) {
+            return sink_launch(sink, name, pf_gemm_bytes(w, n), fn, dim3(pf_grid(g.X, g.Y, g.S)), dim3(NT), 0, g);
+        };
         if (w.fmt == FMT_Q4)
-            return mt == 128  ? q4(k_pf_gemm_q4<2, 4, 4>)
-                   : mt == 64 ? q4(k_pf_gemm_q4<1, 4, 2>)
-                   : mt == 32 ? q4(k_pf_gemm_q4<1, 2, 2>)
-                              : q4(k_pf_gemm_q4<1, 1, 2>);
-        return sink_launch(sink, name, pf_gemm_bytes(w, n), k_pf_gemm_f32, grid, dim3(NT), 0, g);
+            return mt == 128  ? go(k_pf_gemm_q4<2, 4, 4>)
+                   : mt == 64 ? go(k_pf_gemm_q4<1, 4, 2>)
+                   : mt == 32 ? go(k_pf_gemm_q4<1, 2, 2>)
+                              : go(k_pf_gemm_q4<1, 1, 2>);
+        return mt == 64 ? go(k_pf_gemm_f32<4>) : mt == 32 ? go(k_pf_gemm_f32<2>) : go(k_pf_gemm_f32<1>);
     };
     auto rows = [&](const char* name, PfRows r, int n_rows) {
         return with_mg(H, [&](auto mg) {
