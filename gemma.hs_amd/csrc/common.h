@@ -323,9 +323,13 @@ int enqueue_persistent(gh_model* m, gh_kv* kv, Sink& sink, int pos);
 // 135 MB of attention states).
 constexpr int PF_MAX_TOKENS = 2048;
 constexpr int PF_ATTN_NC = 16;      // attention chunks per token and kv head in the prefill
-int pf_tile_rows(int fmt, int n);
+struct PfCut {
+    int mt;   // token rows per workgroup
+    int S;    // column splits
+    int per;  // column blocks per split
+};
 int pf_rows_padded(int fmt, int n);
-int pf_splits(const DMat& w, int n, int* kb_per);
+PfCut pf_cut(const DMat& w, int Pp);
 int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool head);
 int launch_q4_dequant(const DMat& w, float* out, hipStream_t s);
 int launch_matvec_plain(const DMat& w, const Plan& p, const float* x, float* part, float* y,

@@ -4422,7 +4422,8 @@ __device__ __forceinline__ f16x8_t q4_f16x8(uint32_t w0, uint32_t w1, uint32_t b
 //   - the workgroup's A goes through LDS, double-buffered, its loads two
 //     blocks ahead in registers; one barrier per block;
 //   - wave w unpacks the codes and scales of rows 32w .. 32w+31 into LDS a
-//     block ahead, once for the MW waves that use them;
+//     block ahead (loads three blocks ahead), once for the MW waves that use
+//     them;
 //   - 2 chained MFMAs (lo and hi parts) per 16 x 16 subtile into a fresh
 //     accumulator; d * that is added to the sum behind the next subtiles'
 //     MFMAs.
@@ -4473,13 +4474,16 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
     // read that block again and its scales count as zeros, so that a split
     // runs an even number of blocks with no branch between the loads and
     // their use (the compiler would sink them to it).
-    auto load = [&](int j, int i) {
+    auto load_a = [&](int j, int i) {
+        const uint32_t so = 64u * (uint32_t)(kb0 + min(i, nk - 1));
+#pragma unroll
+        for (int q = 0; q < CW; ++q)
+            if (CH >= 4 || wave < CH) ra[j][q] = A.u4s(ao[q], so);
+    };
+    auto load_w = [&](int j, int i) {
         const uint32_t kb = (uint32_t)(kb0 + min(i, nk - 1));
         rb[j] = C.u2s(urow * 16 + 8 * (lane >> 5), kb * TILE_ROWS * 16);
         rs[j] = S.h1s(urow * 2, kb * TILE_ROWS * 2);
-#pragma unroll
-        for (int q = 0; q < CW; ++q)
-            if (CH >= 4 || wave < CH) ra[j][q] = A.u4s(ao[q], 64u * kb);
     };
     const uint32_t bias = pf_bias();
     // block i from slot j into LDS buffer j
@@ -4498,10 +4502,13 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
     for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int n = 0; n < TN; ++n) acc[m][n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    load(0, 0);
-    load(1, 1);
-    unpack(0, 0);
+    load_a(0, 0);
+    load_w(0, 0);
+    load_a(1, 1);
+    load_w(1, 1);
     store_a(0);
+    unpack(0, 0);
+    load_w(0, 2);
     __syncthreads();
     // products of the last token subtiles, added while the next ones' MFMAs run
     f32x4_t cp[TN];
@@ -4528,7 +4535,7 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
                 b[n] = bs[j][r >> 5][kg >> 1][(r & 31) + 32 * (kg & 1)];
                 d[n] = ds[j][r];
             }
-            load(j, i + 2);
+            load_a(j, i + 2);
 #pragma unroll
             for (int m = 0; m < TM; ++m) {
                 f16x8_t an[2] = {a[0], a[1]};
@@ -4548,7 +4555,10 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
                     cp[n] = c[n];
                     dp[n] = d[n];
                 }
-                if (m == TM / 2) unpack(j ^ 1, i + 1);
+                if (m == TM / 2) {
+                    unpack(j ^ 1, i + 1);
+                    load_w(j ^ 1, i + 3);
+                }
                 if (m == TM - 1) store_a(j ^ 1);
                 __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the next operands' reads first
 #pragma unroll
@@ -4979,47 +4989,45 @@ __global__ __launch_bounds__(NT) void k_pf_geglu(const float* part, int ld, int 
     for (int k = 4 * threadIdx.x; k < F; k += 4 * NT) a.put4(t, k, *(const float4*)&rowbuf[k], sc);
 }
 
-// Token rows of one GEMM workgroup for a pass of n tokens, and the pass's rows
-// rounded up to whole workgroups: the smallest tile that holds a short pass
-// (the block time falls with it, see below), else 128 (f32: 64).
-int pf_tile_rows(int fmt, int n) { return n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 || fmt != FMT_Q4 ? 64 : 128; }
+// Rows of a pass of n tokens: rounded up to the largest token tile its GEMMs
+// may take (Q4_0 128, f32 64), or the smallest that holds a short pass.
 int pf_rows_padded(int fmt, int n) {
-    const int mt = pf_tile_rows(fmt, n);
+    const int mt = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 || fmt != FMT_Q4 ? 64 : 128;
     return (n + mt - 1) / mt * mt;
 }
 
-// Split count of a prefill GEMM over a pass of n tokens, at most 8: the S
-// whose estimate is lowest of
-//   rounds of workgroups over the CUs x steps per split x step time
+// Token tile (16, 32, 64; Q4_0 also 128) and split count (at most 8) of a
+// prefill GEMM over a pass of Pp rows: the pair whose estimate is lowest of
+//   rounds of workgroups over the CUs x blocks per split x block time
 //   + the S partials' way out and back in (4 B per row and token each)
-// with what MI355X measured: 0.55 / 0.38 / 0.30 / 0.28 us per 32-column Q4_0
-// block at 128 / 64 / 32 / 16 token rows, 0.55 / 0.33 / 0.21 us per
-// 16-column f32 step at 64 / 32 / 16, 0.58 us per MB of partials.  Over
-// sweeps of S at 16 .. 1907 tokens of the 1B and 4B shapes it picks the best
-// S or one whose GEMM plus consumer is within 3 us of it, but for 1024-token
-// 1B down (3 splits, 62 us with its consumer; 6 take 55).
-int pf_splits(const DMat& w, int n, int* kb_per) {
-    const int mt = pf_tile_rows(w.fmt, n), Pp = pf_rows_padded(w.fmt, n), wgs = w.tiles * (Pp / mt);
+// with what MI355X measured for one workgroup on a CU: 0.28 / 0.30 / 0.38 /
+// 0.55 us per 32-column Q4_0 block at 16 / 32 / 64 / 128 token rows, 0.21 /
+// 0.33 / 0.55 us per 16-column f32 step at 16 / 32 / 64, and 0.58 us per MB of
+// partials.  Over sweeps of S at 16 .. 1907 tokens of the 1B and 4B shapes it
+// picks the best S or one whose GEMM plus consumer is within 3 us of it, but
+// for 1024-token 1B down (3 splits, 62 us with its consumer; 6 take 55).
+PfCut pf_cut(const DMat& w, int Pp) {
+    static const double q4_us[] = {0.28, 0.30, 0.38, 0.55}, f32_us[] = {0.21 / 4, 0.33 / 4, 0.55 / 4};  // per block
     const bool q4 = w.fmt == FMT_Q4;
     // Q4_0: the kernel runs pairs of blocks; f32: steps of 4 blocks, whole rounds of its ring
     const int unit = q4 ? 2 : 4 * PF_F32_DEPTH;
-    auto blocks = [&](int splits) { return ((w.nblk + splits - 1) / splits + unit - 1) / unit * unit; };
-    const double tb = q4 ? (mt == 128 ? 0.55 : mt == 64 ? 0.38 : mt == 32 ? 0.30 : 0.28)
-                         : (mt == 64 ? 0.55 : mt == 32 ? 0.33 : 0.21) / 4;
     // the consumers read all partials through one buffer view (below 2 GiB)
-    const int most = (int)std::max<size_t>(1, std::min<size_t>(8, 0x7fffffffu / ((size_t)4 * Pp * w.tiles * TILE_ROWS)));
-    int S = 1;
-    double best = 0.0;
-    for (int c = 1; c <= std::min(most, w.nblk); ++c) {
-        const double t = (wgs * c + 255) / 256 * blocks(c) * tb + 0.58e-6 * 4.0 * c * Pp * w.tiles * TILE_ROWS;
-        if (c == 1 || t < best) {
-            best = t;
-            S = c;
+    const size_t part = (size_t)4 * Pp * w.tiles * TILE_ROWS;
+    const int most = (int)std::max<size_t>(1, std::min<size_t>(8, 0x7fffffffu / part));
+    PfCut best{};
+    double best_us = 0.0;
+    for (int i = 0; i < (q4 ? 4 : 3) && Pp % (16 << i) == 0; ++i) {
+        for (int S = 1; S <= most; ++S) {
+            const int per = ((w.nblk + S - 1) / S + unit - 1) / unit * unit, used = (w.nblk + per - 1) / per;
+            const double us = (w.tiles * (Pp / (16 << i)) * used + 255) / 256 * per * (q4 ? q4_us[i] : f32_us[i]) +
+                              0.58e-6 * (double)part * used;
+            if (best.mt == 0 || us < best_us) {
+                best = {16 << i, used, per};
+                best_us = us;
+            }
         }
     }
-    const int per = blocks(S);
-    if (kb_per) *kb_per = per;
-    return (w.nblk + per - 1) / per;
+    return best;
 }
 
 static double pf_gemm_bytes(const DMat& w, int n) {
@@ -5030,7 +5038,7 @@ int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool he
     const gh_config& c = m->cfg;
     const PfBufs& B = m->pf;
     const int H = c.hidden, hd = c.head_dim, nkv = c.n_kv_heads, G = c.n_heads / nkv, F = c.ffn;
-    const int Pp = pf_rows_padded(m->fmt, n), mt = pf_tile_rows(m->fmt, n);
+    const int Pp = pf_rows_padded(m->fmt, n);
     if (n <= 0 || Pp > B.cap) return set_error(GH_ERR_INVALID, "internal: prefill of %d rows, buffers hold %d", n, B.cap);
     const int zc = (c.flags & GH_FLAG_ZERO_CENTERED) ? 1 : 0;
     const float eps = c.rms_eps;
@@ -5042,12 +5050,12 @@ int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool he
                          c.n_heads * hd, nkv);
     // GEMM of operand A (K columns) with w into the partials; returns S
     auto gemm = [&](const char* name, const DMat& w, int* S_out) -> int {
-        int per = 0;
-        const int S = pf_splits(w, n, &per);
-        if ((size_t)S * Pp * w.tiles * TILE_ROWS > B.part_floats)
+        const PfCut c = pf_cut(w, Pp);
+        if ((size_t)c.S * Pp * w.tiles * TILE_ROWS > B.part_floats)
             return set_error(GH_ERR_INVALID, "internal: prefill partials too small");
-        *S_out = S;
-        const PfGemm g{A(w.cols), w, per, B.part, w.tiles * TILE_ROWS, w.tiles, Pp / mt, S};
+        *S_out = c.S;
+        const int mt = c.mt;
+        const PfGemm g{A(w.cols), w, c.per, B.part, w.tiles * TILE_ROWS, w.tiles, Pp / mt, c.S};
         auto go = [&](auto fn) {
             return sink_launch(sink, name, pf_gemm_bytes(w, n), fn, dim3(pf_grid(g.X, g.Y, g.S)), dim3(NT), 0, g);
         };

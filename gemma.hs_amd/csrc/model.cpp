@@ -402,8 +402,10 @@ int prefill_reserve(gh_model* m, int n) {
     const size_t kmax = std::max({(size_t)H, (size_t)nq * hd, (size_t)c.ffn});
     size_t part = 0;
     for (const DMat* w : {&L.qkv, &L.o, &L.gu, &L.down})
-        for (int k = 16; k <= cap; k += 16)
-            part = std::max(part, (size_t)pf_splits(*w, k, nullptr) * pf_rows_padded(w->fmt, k) * w->tiles * TILE_ROWS);
+        for (int k = 16; k <= cap; k += 16) {
+            const int pp = pf_rows_padded(w->fmt, k);
+            part = std::max(part, (size_t)pf_cut(*w, pp).S * pp * w->tiles * TILE_ROWS);
+        }
     PfBufs& B = m->pf;
     auto get = [&](void** p, size_t bytes) -> int {
         hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));
