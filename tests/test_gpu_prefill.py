@@ -210,6 +210,47 @@ def test_prefill_gemm_tile_edges(ctx, n):
     assert rel_err(la, lb) < ACT_TOL and na == nb
 
 
+@pytest.mark.parametrize("n", [2, 16, 17, 33, 64, 65, 130])
+def test_prefill_f32_gemm_tile_edges(ctx, n):
+    """f32 prefill GEMM at the edges of its token tiles (16, 32, 64 rows)
+    and of its rounds of column steps (hidden 288: 18 steps, ffn 352: 22):
+    as the Q4_0 test above, with its bound."""
+    cfg = _mini4b(gh.MODE_GEMMA3, window=40, layers=2)
+    cfg.hidden, cfg.ffn, cfg.max_seq = 288, 352, 144
+    m = _gpu_model(ctx, cfg, 37, False)
+    toks = gh.synth_tokens(15, "f32tile", n, cfg.vocab)
+    kv_a, kv_b = gh.KVCache(m, 144), gh.KVCache(m, 144)
+    la, ya, na = gh.prefill(m, kv_a, toks, want_layers=True)
+    for t in toks[:-1]:
+        gh.runGemmaInferenceCached(m, int(t), kv_b, want_logits=False)
+    lb, _, yb, nb = gh.runGemmaInferenceCachedWithLayer0(m, int(toks[-1]), kv_b)
+    for l in range(cfg.n_layers):
+        assert rel_err(ya[l], yb[l]) < ACT_TOL, l
+    assert rel_err(la, lb) < ACT_TOL and na == nb
+
+
+@pytest.mark.parametrize("nq,nkv", [(4, 4), (8, 4), (4, 1), (8, 1)])
+@pytest.mark.parametrize("n", [16, 97, 300])
+def test_prefill_attention_chunks_outside_the_window(ctx, nq, nkv, n):
+    """Chunk states of the matrix-core attention and their merge, per GQA
+    group, at one chunk, at shared chunks of 16 positions and past 16 of them
+    (300 tokens: 32-position chunks, most outside a 20-position window):
+    every layer of the last token against the decode step, ACT_TOL as
+    above."""
+    cfg = _mini4b(gh.MODE_GEMMA3, window=20, layers=2)
+    cfg.n_heads, cfg.n_kv_heads, cfg.max_seq = nq, nkv, 304
+    m = _gpu_model(ctx, cfg, 41, True)
+    toks = gh.synth_tokens(16, "chunk", n, cfg.vocab)
+    kv_a, kv_b = gh.KVCache(m, 304), gh.KVCache(m, 304)
+    la, ya, na = gh.prefill(m, kv_a, toks, want_layers=True)
+    for t in toks[:-1]:
+        gh.runGemmaInferenceCached(m, int(t), kv_b, want_logits=False)
+    lb, _, yb, nb = gh.runGemmaInferenceCachedWithLayer0(m, int(toks[-1]), kv_b)
+    for l in range(cfg.n_layers):
+        assert rel_err(ya[l], yb[l]) < ACT_TOL, l
+    assert rel_err(la, lb) < ACT_TOL and na == nb
+
+
 def test_prefill_single_token_equals_step(ctx):
     """A prefill of one token is the decode step of that token."""
     cfg = _mini4b(gh.MODE_GEMMA3, layers=2)
