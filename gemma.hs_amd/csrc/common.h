@@ -328,6 +328,7 @@ struct PfCut {
     int S;    // column splits
     int per;  // column blocks per split
 };
+constexpr int PF_F32_DEPTH = 4;  // 16-column steps in flight in the f32 prefill GEMM
 int pf_rows_padded(int fmt, int n);
 PfCut pf_cut(const DMat& w, int Pp);
 int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool head);

@@ -4604,7 +4604,6 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
 // below that of one chain over all the columns.  1B shape, 300 tokens: gate/up
 // 709 -> 117 us (82 TFLOP/s; the f32 matrix peak this card reaches is 138), down
 // 424 -> 72; the kernel before it waited on one load per MFMA.
-constexpr int PF_F32_DEPTH = 4;
 template <int TM>
 __global__ __launch_bounds__(NT, 2) void k_pf_gemm_f32(PfGemm g) {
     constexpr int TN = 2, MT = 16 * TM, D = PF_F32_DEPTH;
@@ -5019,47 +5018,6 @@ __global__ __launch_bounds__(NT) void k_pf_geglu(const float* part, int ld, int 
     }
     const float sc = a.row_scale(t, block_max(mx, slot));  // barrier: rowbuf complete
     for (int k = 4 * threadIdx.x; k < F; k += 4 * NT) a.put4(t, k, *(const float4*)&rowbuf[k], sc);
-}
-
-// Rows of a pass of n tokens: rounded up to the largest token tile its GEMMs
-// may take (Q4_0 128, f32 64), or the smallest that holds a short pass.
-int pf_rows_padded(int fmt, int n) {
-    const int mt = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 || fmt != FMT_Q4 ? 64 : 128;
-    return (n + mt - 1) / mt * mt;
-}
-
-// Token tile (16, 32, 64; Q4_0 also 128) and split count (at most 8) of a
-// prefill GEMM over a pass of Pp rows: the pair whose estimate is lowest of
-//   rounds of workgroups over the CUs x blocks per split x block time
-//   + the S partials' way out and back in (4 B per row and token each)
-// with what MI355X measured for one workgroup on a CU: 0.28 / 0.30 / 0.38 /
-// 0.55 us per 32-column Q4_0 block at 16 / 32 / 64 / 128 token rows, 0.21 /
-// 0.33 / 0.55 us per 16-column f32 step at 16 / 32 / 64, and 0.58 us per MB of
-// partials.  Over sweeps of S at 16 .. 1907 tokens of the 1B and 4B shapes it
-// picks the best S or one whose GEMM plus consumer is within 3 us of it, but
-// for 1024-token 1B down (3 splits, 62 us with its consumer; 6 take 55).
-PfCut pf_cut(const DMat& w, int Pp) {
-    static const double q4_us[] = {0.28, 0.30, 0.38, 0.55}, f32_us[] = {0.21 / 4, 0.33 / 4, 0.55 / 4};  // per block
-    const bool q4 = w.fmt == FMT_Q4;
-    // Q4_0: the kernel runs pairs of blocks; f32: steps of 4 blocks, whole rounds of its ring
-    const int unit = q4 ? 2 : 4 * PF_F32_DEPTH;
-    // the consumers read all partials through one buffer view (below 2 GiB)
-    const size_t part = (size_t)4 * Pp * w.tiles * TILE_ROWS;
-    const int most = (int)std::max<size_t>(1, std::min<size_t>(8, 0x7fffffffu / part));
-    PfCut best{};
-    double best_us = 0.0;
-    for (int i = 0; i < (q4 ? 4 : 3) && Pp % (16 << i) == 0; ++i) {
-        for (int S = 1; S <= most; ++S) {
-            const int per = ((w.nblk + S - 1) / S + unit - 1) / unit * unit, used = (w.nblk + per - 1) / per;
-            const double us = (w.tiles * (Pp / (16 << i)) * used + 255) / 256 * per * (q4 ? q4_us[i] : f32_us[i]) +
-                              0.58e-6 * (double)part * used;
-            if (best.mt == 0 || us < best_us) {
-                best = {16 << i, used, per};
-                best_us = us;
-            }
-        }
-    }
-    return best;
 }
 
 static double pf_gemm_bytes(const DMat& w, int n) {
