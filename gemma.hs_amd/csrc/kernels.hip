@@ -4425,8 +4425,16 @@ __device__ __forceinline__ f16x8_t q4_f16x8(uint32_t w0, uint32_t w1, uint32_t b
 //     block ahead (loads three blocks ahead), once for the MW waves that use
 //     them;
 //   - 2 chained MFMAs (lo and hi parts) per 16 x 16 subtile into a fresh
-//     accumulator; d * that is added to the sum behind the next subtiles'
-//     MFMAs.
+//     accumulator; d * that is added to the run's sum behind the next
+//     subtiles' MFMAs;
+//   - every PF_RUN blocks the run's sum goes to the running one and starts
+//     from zero: the rounding error of 72 blocks (1907 tokens of 1B, down) is
+//     that of sums of 8 and of 9, not of one chain.  Logits' error against 64
+//     bits, one chain / runs of 8: 8.7e-7 / 7.4e-7 there, 6.6e-7 / 5.9e-7 at
+//     4B 1024 tokens.  It takes 2 to 2.7 % of a prefill (1907 tokens 11.14 ->
+//     11.46 ms); runs of 16 would leave o_proj's sum of 32 blocks longer than
+//     its 4 splits of 8 once were.  Unrolling the run to put its adds between
+//     the MFMAs spills (91 VGPRs).
 // The 128 x 128 tile takes 0.55 us per block and CU, whether one or two
 // workgroups share the CU: per wave 32 MFMAs (512 cycles), 95 VALU
 // instructions (64 of them the scale FMAs) and 20 LDS ones.  Four blocks in
@@ -4435,6 +4443,7 @@ __device__ __forceinline__ f16x8_t q4_f16x8(uint32_t w0, uint32_t w1, uint32_t b
 // replaced (16 tokens a wave, whose LDS reads took as long as its MFMAs), 512
 // tokens: 1B gate/up 49 -> 43 us, 4B gate/up 135 -> 122, qkv 45 -> 30, down
 // 79 -> 66.
+constexpr int PF_RUN = 8;  // column blocks a sum runs over (even)
 template <int MW, int TM, int TN>
 __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
     constexpr int NW = 4 / MW, MT = 16 * TM * MW;
@@ -4518,64 +4527,79 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
         cp[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         dp[n] = 0.0f;
     }
-    for (int base = 0; base < nk; base += 2) {
+    f32x4_t sum[TM][TN];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int i = base + j;
-            auto read_a = [&](int m, int p) {
-                return __builtin_bit_cast(f16x8_t, as[j][p * (MT / 16) + wm * TM + m][m16 * 4 + (kg ^ f(m16))]);
-            };
-            f16x8_t b[TN], a[2];
-            float d[TN];
-            a[1] = read_a(0, 1);
-            a[0] = read_a(0, 0);
+    for (int m = 0; m < TM; ++m)
 #pragma unroll
-            for (int n = 0; n < TN; ++n) {
-                const int r = 16 * (TN * wn + n) + m16;
-                b[n] = bs[j][r >> 5][kg >> 1][(r & 31) + 32 * (kg & 1)];
-                d[n] = ds[j][r];
-            }
-            load_a(j, i + 2);
+        for (int n = 0; n < TN; ++n) sum[m][n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int run = 0; run < nk; run += PF_RUN) {
+        const int end = min(nk, run + PF_RUN);
+        for (int base = run; base < end; base += 2) {
 #pragma unroll
-            for (int m = 0; m < TM; ++m) {
-                f16x8_t an[2] = {a[0], a[1]};
-                if (m + 1 < TM) {
-                    an[1] = read_a(m + 1, 1);
-                    an[0] = read_a(m + 1, 0);
-                }
-                f32x4_t c[TN];
-#pragma unroll
-                for (int n = 0; n < TN; ++n)
-                    c[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[1], b[n], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                for (int n = 0; n < TN; ++n) c[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[n], c[n], 0, 0, 0);
+            for (int j = 0; j < 2; ++j) {
+                const int i = base + j;
+                auto read_a = [&](int m, int p) {
+                    return __builtin_bit_cast(f16x8_t, as[j][p * (MT / 16) + wm * TM + m][m16 * 4 + (kg ^ f(m16))]);
+                };
+                f16x8_t b[TN], a[2];
+                float d[TN];
+                a[1] = read_a(0, 1);
+                a[0] = read_a(0, 0);
 #pragma unroll
                 for (int n = 0; n < TN; ++n) {
-                    acc[(m + TM - 1) % TM][n] += dp[n] * cp[n];
-                    cp[n] = c[n];
-                    dp[n] = d[n];
+                    const int r = 16 * (TN * wn + n) + m16;
+                    b[n] = bs[j][r >> 5][kg >> 1][(r & 31) + 32 * (kg & 1)];
+                    d[n] = ds[j][r];
                 }
-                if (m == TM / 2) {
-                    unpack(j ^ 1, i + 1);
-                    load_w(j ^ 1, i + 3);
-                }
-                if (m == TM - 1) store_a(j ^ 1);
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the next operands' reads first
+                load_a(j, i + 2);
 #pragma unroll
-                for (int t = 0; t < 2 * TN; ++t) {  // then VALU work between the MFMAs
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                for (int m = 0; m < TM; ++m) {
+                    f16x8_t an[2] = {a[0], a[1]};
+                    if (m + 1 < TM) {
+                        an[1] = read_a(m + 1, 1);
+                        an[0] = read_a(m + 1, 0);
+                    }
+                    f32x4_t c[TN];
+#pragma unroll
+                    for (int n = 0; n < TN; ++n)
+                        c[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[1], b[n], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                    for (int n = 0; n < TN; ++n) c[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[n], c[n], 0, 0, 0);
+#pragma unroll
+                    for (int n = 0; n < TN; ++n) {
+                        acc[(m + TM - 1) % TM][n] += dp[n] * cp[n];
+                        cp[n] = c[n];
+                        dp[n] = d[n];
+                    }
+                    if (m == TM / 2) {
+                        unpack(j ^ 1, i + 1);
+                        load_w(j ^ 1, i + 3);
+                    }
+                    if (m == TM - 1) store_a(j ^ 1);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the next operands' reads first
+#pragma unroll
+                    for (int t = 0; t < 2 * TN; ++t) {  // then VALU work between the MFMAs
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    a[0] = an[0];
+                    a[1] = an[1];
                 }
+                __syncthreads();
                 __builtin_amdgcn_sched_barrier(0);
-                a[0] = an[0];
-                a[1] = an[1];
             }
-            __syncthreads();
-            __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int n = 0; n < TN; ++n) {
+                sum[m][n] += acc[m][n];
+                acc[m][n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
     }
 #pragma unroll
-    for (int n = 0; n < TN; ++n) acc[TM - 1][n] += dp[n] * cp[n];
+    for (int n = 0; n < TN; ++n) sum[TM - 1][n] += dp[n] * cp[n];
     // lane holds weight row 16 n + m16 of the wave's, tokens 4 kg .. 4 kg + 3 of each 16
 #pragma unroll
     for (int m = 0; m < TM; ++m) {
@@ -4584,10 +4608,10 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
         float* o = g.out + ((size_t)pt.z * g.a.Pp + tw) * g.ldo + (size_t)pt.x * TILE_ROWS + 16 * TN * wn + m16;
 #pragma unroll
         for (int n = 0; n < TN; ++n) {
-            o[16 * n] = acc[m][n][0] * inv.x;
-            o[(size_t)g.ldo + 16 * n] = acc[m][n][1] * inv.y;
-            o[2 * (size_t)g.ldo + 16 * n] = acc[m][n][2] * inv.z;
-            o[3 * (size_t)g.ldo + 16 * n] = acc[m][n][3] * inv.w;
+            o[16 * n] = sum[m][n][0] * inv.x;
+            o[(size_t)g.ldo + 16 * n] = sum[m][n][1] * inv.y;
+            o[2 * (size_t)g.ldo + 16 * n] = sum[m][n][2] * inv.z;
+            o[3 * (size_t)g.ldo + 16 * n] = sum[m][n][3] * inv.w;
         }
     }
 }

@@ -229,6 +229,71 @@ def test_prefill_f32_gemm_tile_edges(ctx, n):
     assert rel_err(la, lb) < ACT_TOL and na == nb
 
 
+def _q4_rows(rows, code_blocks, scales):
+    """GGUF Q4_0 bytes of `rows` equal rows: per block 32 codes and an fp16 scale."""
+    d = np.asarray(scales, np.float16).reshape(-1, 1).view(np.uint8)
+    q = np.asarray(code_blocks, np.uint8)
+    row = np.concatenate([d, q[:, :16] | (q[:, 16:] << 4)], axis=1).reshape(-1)
+    return np.tile(row, (rows, 1))
+
+
+@pytest.mark.parametrize("hidden,ffn,n", [(1152, 6912, 37), (1152, 6912, 257), (1152, 6912, 1907),
+                                          (2560, 10240, 1024)])
+def test_prefill_q4_sums_restart(ctx, hidden, ffn, n):
+    """The Q4_0 GEMM's f32 sums are restarted every 8 column blocks, so the
+    down projection's error stays that of short sums.
+
+    gate and up have equal rows, so h is one value in all ffn columns.  Even
+    rows of down hold -4096 h in block 0 and 0.45 ulp of that in each other
+    block; odd rows hold block 0 only.  Every product is exact.  One chain
+    loses each small term that follows the large one (32 ulp over 72
+    blocks).  Sums of 8 blocks, each added to a running one, round at most
+    8 + nblk / 8 times, the split partials and the residual 8 + 1 times more:
+    half an ulp each."""
+    cfg = gh.preset("gemma3-1b")
+    cfg.vocab, cfg.hidden, cfg.ffn, cfg.n_layers, cfg.max_seq = 64, hidden, ffn, 1, 2048
+    cfg.flags &= ~gh.FLAG_POST_FFN_NORM
+    nh, nf, one = hidden // 32, ffn // 32, np.float16(1.0)
+    zero, ones = np.full((1, 32), 8), np.full((1, 32), 9)
+    m = gh.GemmaModel(ctx, cfg)
+
+    def mat(name, rows):
+        m.set_tensor(name, np.ascontiguousarray(rows).reshape(-1), gh.DTYPE_Q4_0)
+
+    def quiet(rows, nblk):
+        return _q4_rows(rows, np.tile(zero, (nblk, 1)), np.full(nblk, one))
+
+    mat("token_embd.weight", _q4_rows(64, np.tile(ones, (nh, 1)), np.full(nh, 2.0 ** -10)))
+    m.set_tensor("output_norm.weight", np.ones(hidden, np.float32), gh.DTYPE_F32)
+    for name, rows, nblk in (("attn_q", 1024, nh), ("attn_k", 256, nh), ("attn_v", 256, nh), ("attn_output", hidden, 32)):
+        mat("blk.0.%s.weight" % name, quiet(rows, nblk))
+    for name, k in (("attn_norm", hidden), ("attn_q_norm", 256), ("attn_k_norm", 256), ("post_attention_norm", hidden),
+                    ("ffn_norm", hidden), ("post_ffw_norm", hidden)):
+        m.set_tensor("blk.0.%s.weight" % name, np.ones(k, np.float32), gh.DTYPE_F32)
+    for name in ("ffn_gate", "ffn_up"):
+        mat("blk.0.%s.weight" % name, _q4_rows(ffn, np.tile(ones, (nh, 1)), np.full(nh, 0.003)))
+    a = hidden * float(np.float16(0.003)) * (2.0 if cfg.flags & gh.FLAG_ZERO_CENTERED else 1.0)
+    h = 0.5 * a * (1.0 + np.tanh(min(0.7978845608 * (a + 0.044715 * a ** 3), 10.0))) * a
+    tiny = np.float16(0.45 * float(np.spacing(np.float32(4096.0 * h))) / h)
+    codes, scales = np.full((nf, 32), 8), np.full(nf, one)
+    codes[0], scales[0] = 0, np.float16(16.0)  # -8 * 32 * 16 = -4096
+    odd = _q4_rows(hidden // 2, codes, scales)
+    codes[1:, 5], scales[1:] = 7, tiny
+    down = np.empty((hidden, nf * 18), np.uint8)
+    down[0::2], down[1::2] = _q4_rows(hidden // 2, codes, scales), odd
+    mat("blk.0.ffn_down.weight", down)
+
+    _, layers, _ = gh.prefill(m, gh.KVCache(m, 2048), np.zeros(n, np.int32), want_logits=False, want_layers=True)
+    out = layers[0].astype(np.float64)
+    big = out[1]
+    assert big < -1000.0 and np.ptp(out[0::2]) == 0.0 and np.ptp(out[1::2]) == 0.0
+    ulp = float(np.spacing(np.float32(abs(big))))
+    small = big * float(tiny) / 4096.0  # a block's term (the residual's share of `big` is below 1e-5)
+    assert 0.43 < abs(small) / ulp < 0.47
+    err = abs((out[0] - big) - (nf - 1) * small) / ulp
+    assert err <= 0.5 * (8 + nf / 8 + 8 + 1), (err, small / ulp)
+
+
 @pytest.mark.parametrize("nq,nkv", [(4, 4), (8, 4), (4, 1), (8, 1)])
 @pytest.mark.parametrize("n", [16, 97, 300])
 def test_prefill_attention_chunks_outside_the_window(ctx, nq, nkv, n):
