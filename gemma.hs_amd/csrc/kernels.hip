@@ -4623,14 +4623,15 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
 // MFMA e of the step multiplies element e of both (the sum runs over every
 // column once, in that order).  At 64 x 32 per wave six loads feed 32 MFMAs
 // of 32 cycles, so operands come straight from L1/L2, PF_F32_DEPTH steps
-// ahead, with no LDS and no barrier.  Each PF_F32_DEPTH steps are summed from
-// zero and then added to the running sum, which keeps the rounding error
-// below that of one chain over all the columns.  1B shape, 300 tokens: gate/up
+// ahead, with no LDS and no barrier.  Each RUN steps are summed from zero and
+// then added to the running sum, which keeps the rounding error below that of
+// one chain over all the columns.  1B shape, 300 tokens: gate/up
 // 709 -> 117 us (82 TFLOP/s; the f32 matrix peak this card reaches is 138), down
 // 424 -> 72; the kernel before it waited on one load per MFMA.
-template <int TM>
+template <int TM, int RUN>
 __global__ __launch_bounds__(NT, 2) void k_pf_gemm_f32(PfGemm g) {
     constexpr int TN = 2, MT = 16 * TM, D = PF_F32_DEPTH;
+    static_assert(D % RUN == 0, "a round of the ring is whole runs");
     PfTile pt;
     if (!pf_tile(g, pt)) return;  // uniform per workgroup
     const int wave = wave_id(), lane = threadIdx.x & 63, i16 = lane & 15, q = lane >> 4;
@@ -4666,14 +4667,16 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_f32(PfGemm g) {
 #pragma unroll
                     for (int n = 0; n < TN; ++n)
                         c[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                            ra[j][m][e], rb[j][n][e], j + e ? c[m][n] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                            ra[j][m][e], rb[j][n][e], j % RUN + e ? c[m][n] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
             load(j, base + D + j);
+            if ((j + 1) % RUN == 0) {
+#pragma unroll
+                for (int m = 0; m < TM; ++m)
+#pragma unroll
+                    for (int n = 0; n < TN; ++n) acc[m][n] += c[m][n];
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int m = 0; m < TM; ++m)
-#pragma unroll
-            for (int n = 0; n < TN; ++n) acc[m][n] += c[m][n];
     }
     // lane holds weight row 32 wave + 16 n + i16 of the tile, tokens 4 q .. 4 q + 3 of each 16
     float* o = g.out + ((size_t)pt.z * g.a.Pp + t0 + 4 * q) * g.ldo + (size_t)pt.x * TILE_ROWS + 32 * wave + i16;
@@ -5078,7 +5081,14 @@ int enqueue_prefill(gh_model* m, gh_kv* kv, Sink& sink, int n, int pos0, bool he
                    : mt == 64 ? go(k_pf_gemm_q4<1, 4, 2>)
                    : mt == 32 ? go(k_pf_gemm_q4<1, 2, 2>)
                               : go(k_pf_gemm_q4<1, 1, 2>);
-        return mt == 64 ? go(k_pf_gemm_f32<4>) : mt == 32 ? go(k_pf_gemm_f32<2>) : go(k_pf_gemm_f32<1>);
+        // Sums of 64 columns, or of 16 below 512 columns: there 64 make up a
+        // large part of the whole.  Logits' error against 64 bits of the tiny
+        // model (128 and 512 columns), sums of 64 / 16: 5.2e-7 / 4.0e-7.  At
+        // 1152 to 6912 columns: 7.3e-7 to 7.7e-7 / 6.1e-7 to 7.3e-7 for 1 to 4
+        // % more time (300 tokens 1.80 -> 1.86 ms), so those keep 64.
+        if (w.cols < 512)
+            return mt == 64 ? go(k_pf_gemm_f32<4, 1>) : mt == 32 ? go(k_pf_gemm_f32<2, 1>) : go(k_pf_gemm_f32<1, 1>);
+        return mt == 64 ? go(k_pf_gemm_f32<4, 4>) : mt == 32 ? go(k_pf_gemm_f32<2, 4>) : go(k_pf_gemm_f32<1, 4>);
     };
     auto rows = [&](const char* name, PfRows r, int n_rows) {
         return with_mg(H, [&](auto mg) {

@@ -294,6 +294,44 @@ def test_prefill_q4_sums_restart(ctx, hidden, ffn, n):
     assert err <= 0.5 * (8 + nf / 8 + 8 + 1), (err, small / ulp)
 
 
+@pytest.mark.parametrize("ffn,n", [(128, 37), (256, 300), (480, 70)])
+def test_prefill_f32_sums_restart(ctx, ffn, n):
+    """Below 512 columns the f32 GEMM's sums are restarted every 16: as in the
+    Q4_0 test above, down's even rows hold -4096 h in column 0 and 0.45 ulp
+    of that in each other column.  A chain of 64 columns loses 28 ulp; sums
+    of 16, each added to the split's running one, round at most 16 +
+    columns / 16 times with the splits, the residual once or twice more."""
+    cfg = gh.preset("tiny")
+    cfg.vocab, cfg.ffn, cfg.n_layers = 64, ffn, 1
+    cfg.flags &= ~gh.FLAG_POST_FFN_NORM
+    m = gh.GemmaModel(ctx, cfg)
+    H, q = cfg.hidden, cfg.n_heads * cfg.head_dim
+    kv = cfg.n_kv_heads * cfg.head_dim
+    down = np.zeros((H, ffn), np.float32)
+    a = H * float(np.float32(0.02)) * (2.0 if cfg.flags & gh.FLAG_ZERO_CENTERED else 1.0)
+    h = 0.5 * a * (1.0 + np.tanh(min(0.7978845608 * (a + 0.044715 * a ** 3), 10.0))) * a
+    tiny = np.float32(0.45 * float(np.spacing(np.float32(4096.0 * h))) / h)
+    down[0::2, 1:] = -tiny
+    down[:, 0] = -4096.0
+    for name, t in (("token_embd", np.full((64, H), 2.0 ** -10)), ("output_norm", np.ones(H)),
+                    ("blk.0.attn_q", np.zeros((q, H))), ("blk.0.attn_k", np.zeros((kv, H))),
+                    ("blk.0.attn_v", np.zeros((kv, H))), ("blk.0.attn_output", np.zeros((H, q))),
+                    ("blk.0.ffn_gate", np.full((ffn, H), 0.02)), ("blk.0.ffn_up", np.full((ffn, H), 0.02)),
+                    ("blk.0.ffn_down", down), ("blk.0.attn_norm", np.ones(H)), ("blk.0.ffn_norm", np.ones(H)),
+                    ("blk.0.attn_q_norm", np.ones(cfg.head_dim)), ("blk.0.attn_k_norm", np.ones(cfg.head_dim)),
+                    ("blk.0.post_attention_norm", np.ones(H)), ("blk.0.post_ffw_norm", np.ones(H))):
+        m.set_tensor(name + ".weight", t.astype(np.float32).reshape(-1), gh.DTYPE_F32)
+    _, layers, _ = gh.prefill(m, gh.KVCache(m, 512), np.zeros(n, np.int32), want_logits=False, want_layers=True)
+    out = layers[0].astype(np.float64)
+    big = out[1]
+    assert big < -1000.0 and np.ptp(out[0::2]) == 0.0 and np.ptp(out[1::2]) == 0.0
+    ulp = float(np.spacing(np.float32(abs(big))))
+    small = big * float(tiny) / 4096.0
+    assert 0.43 < abs(small) / ulp < 0.47
+    err = abs((out[0] - big) - (ffn - 1) * small) / ulp
+    assert err <= 0.5 * (16 + ffn / 16 + 2), (err, small / ulp)
+
+
 @pytest.mark.parametrize("nq,nkv", [(4, 4), (8, 4), (4, 1), (8, 1)])
 @pytest.mark.parametrize("n", [16, 97, 300])
 def test_prefill_attention_chunks_outside_the_window(ctx, nq, nkv, n):
