@@ -434,14 +434,9 @@ void free_prefill(gh_model* m) {
     B = PfBufs{};
 }
 
-// Prefill buffers for passes of up to n tokens (rows rounded up to 128).
-int prefill_reserve(gh_model* m, int n) {
+// Prefill buffers of `cap` token rows (a multiple of 128), none held before.
+int prefill_alloc(gh_model* m, int cap) {
     const gh_config& c = m->cfg;
-    const int cap = (n + 127) / 128 * 128;
-    if (cap > PF_MAX_TOKENS) return set_error(GH_ERR_INVALID, "internal: prefill pass of %d tokens", n);
-    if (m->pf.cap >= cap) return GH_OK;
-    GH_HIP(hipStreamSynchronize(m->ctx->stream));
-    free_prefill(m);
     const LayerDev& L = m->layers[0];
     const int H = c.hidden, nq = c.n_heads, hd = c.head_dim;
     const size_t kmax = std::max({(size_t)H, (size_t)nq * hd, (size_t)c.ffn});
@@ -455,6 +450,7 @@ int prefill_reserve(gh_model* m, int n) {
     auto get = [&](void** p, size_t bytes) -> int {
         hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));
         if (e != hipSuccess) {
+            (void)hipGetLastError();  // not a later launch's error
             free_prefill(m);
             return set_error(GH_ERR_OOM, "prefill: hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
         }
@@ -471,6 +467,22 @@ int prefill_reserve(gh_model* m, int n) {
     B.part_floats = part;
     B.cap = cap;
     return GH_OK;
+}
+
+// Prefill buffers for a prompt of n tokens: one pass of up to PF_MAX_TOKENS,
+// or passes of 1024 or 512 where the longer one's buffers (332 MB for 2048
+// tokens of the 1B shape, 581 of the 4B shape) do not fit in the device.
+int prefill_reserve(gh_model* m, int n) {
+    int cap = (std::min(n, PF_MAX_TOKENS) + 127) / 128 * 128;
+    if (m->pf.cap >= cap) return GH_OK;
+    GH_HIP(hipStreamSynchronize(m->ctx->stream));
+    free_prefill(m);
+    int rc = prefill_alloc(m, cap);
+    while (rc == GH_ERR_OOM && cap > 512) {
+        cap = cap > 1024 ? 1024 : 512;
+        rc = prefill_alloc(m, cap);
+    }
+    return rc;
 }
 
 int model_check(const gh_model* m);
@@ -1595,7 +1607,7 @@ static int collect_stats(Profiler& prof, gh_kernel_stat* stats, int32_t max_stat
 }
 
 // Batched prefill of n tokens at the cache's next positions, in passes of
-// up to PF_MAX_TOKENS; the last token's logits, layer outputs and next token
+// up to the buffers' rows; the last token's logits, layer outputs and next token
 // are those of gh_step at that position.
 static int prefill_run(gh_model* m, gh_kv* kv, const int32_t* tokens, int32_t n, float* logits, float* layer_out,
                        int32_t* next_out, Profiler* prof = nullptr) {
@@ -1607,13 +1619,13 @@ static int prefill_run(gh_model* m, gh_kv* kv, const int32_t* tokens, int32_t n,
     if ((long long)kv->len + n > kv->max_seq)
         return set_error(GH_ERR_RANGE, "prefill of %d tokens from position %d; KV holds %d", n, kv->len, kv->max_seq);
     hipStream_t s = m->ctx->stream;
-    GH_CHECK(prefill_reserve(m, std::min(n, PF_MAX_TOKENS)));
+    GH_CHECK(prefill_reserve(m, n));
     GH_CHECK(put_state(kv, kv->len + n - 1, tokens[n - 1], kv->len, 0, 0));
     Sink sink;
     sink.s = s;
     sink.prof = prof;
     for (int done = 0; done < n;) {
-        const int k = std::min(PF_MAX_TOKENS, n - done);
+        const int k = std::min(m->pf.cap, n - done);
         GH_HIP(hipMemcpyAsync(m->pf.tok, tokens + done, sizeof(int32_t) * k, hipMemcpyHostToDevice, s));
         GH_CHECK(enqueue_prefill(m, kv, sink, k, kv->len + done, done + k == n));
         done += k;

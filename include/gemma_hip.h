@@ -294,7 +294,8 @@ int gh_generate(gh_model* m, gh_kv* kv, const int32_t* prompt, int32_t n_prompt,
  * call (src/Gemma/Model.hs:1321-1324).
  * The n tokens run at the cache's next positions in one pass per layer:
  * the projections are Q4_0 (or f32) GEMMs on MFMA, attention is causal
- * over the cache, and K/V are appended.  Passes hold up to 2048 tokens.
+ * over the cache, and K/V are appended.  Passes hold up to 2048 tokens, or
+ * 1024 or 512 where the device memory does not hold a longer one's buffers.
  * The cache then holds n more positions.  logits[vocab], layer_out
  * [n_layers*hidden] (may be NULL) and next_out (greedy, or sampled per
  * gh_kv_set_sampling) are those of the last token: what gh_step on that

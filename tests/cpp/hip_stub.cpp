@@ -12,8 +12,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <mutex>
-#include <set>
 
 namespace {
 
@@ -27,10 +27,11 @@ std::mutex& mu() {
     static auto* m = new std::mutex();
     return *m;
 }
-std::set<void*>& live_allocs() {
-    static auto* s = new std::set<void*>();
+std::map<void*, size_t>& live_allocs() {
+    static auto* s = new std::map<void*, size_t>();
     return *s;
 }
+size_t live_bytes = 0, device_bytes = SIZE_MAX;
 
 // Reads the object's first word: a use-after-free under AddressSanitizer.
 hipError_t touch(const void* o, unsigned magic) {
@@ -42,9 +43,11 @@ void* obj(unsigned magic) { return new StubObj{magic}; }
 
 hipError_t dev_alloc(void** p, size_t n) {
     if (!p) return hipErrorInvalidValue;
-    *p = std::malloc(n ? n : 1);
     std::lock_guard<std::mutex> g(mu());
-    live_allocs().insert(*p);
+    if (n > device_bytes || live_bytes > device_bytes - n) return hipErrorOutOfMemory;
+    *p = std::malloc(n ? n : 1);
+    live_allocs()[*p] = n;
+    live_bytes += n;
     return hipSuccess;
 }
 
@@ -52,10 +55,13 @@ hipError_t dev_free(void* p) {
     if (!p) return hipSuccess;
     {
         std::lock_guard<std::mutex> g(mu());
-        if (!live_allocs().erase(p)) {
+        auto it = live_allocs().find(p);
+        if (it == live_allocs().end()) {
             std::fprintf(stderr, "hip_stub: free of a pointer that is not a live allocation: %p\n", p);
             std::abort();
         }
+        live_bytes -= it->second;
+        live_allocs().erase(it);
     }
     std::free(p);
     return hipSuccess;
@@ -64,6 +70,16 @@ hipError_t dev_free(void* p) {
 }  // namespace
 
 extern "C" {
+
+// The device's memory, for tests of what a call does when it runs out.
+size_t hip_stub_live_bytes(void) {
+    std::lock_guard<std::mutex> g(mu());
+    return live_bytes;
+}
+void hip_stub_set_device_bytes(size_t n) {
+    std::lock_guard<std::mutex> g(mu());
+    device_bytes = n;
+}
 
 hipError_t hipGetDeviceCount(int* n) {
     *n = 1;

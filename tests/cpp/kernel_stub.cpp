@@ -16,11 +16,11 @@ int persistent_supported(const gh_model*) { return 0; }
 int enqueue_persistent(gh_model*, gh_kv*, Sink&, int) { return GH_OK; }
 size_t persistent_land(const gh_model*) { return 0; }
 int launch_interleave_gu(const DMat&, int, int, const DMat&, hipStream_t) { return GH_OK; }
-int pf_splits(const DMat&, int, int* kb_per) {
-    if (kb_per) *kb_per = 1;
-    return 1;
+std::vector<int> prefill_passes;  // tokens of every prefill pass, in order
+int enqueue_prefill(gh_model* m, gh_kv*, Sink&, int n, int, bool) {
+    prefill_passes.push_back(n);
+    return n <= m->pf.cap ? GH_OK : GH_ERR_INVALID;
 }
-int enqueue_prefill(gh_model*, gh_kv*, Sink&, int, int, bool) { return GH_OK; }
 int launch_q4_dequant(const DMat&, float*, hipStream_t) { return GH_OK; }
 int launch_matvec_plain(const DMat&, const Plan&, const float*, float*, float*, int, float, hipStream_t) { return GH_OK; }
 int launch_rmsnorm(const float*, const float*, int, float, int, float*, hipStream_t) { return GH_OK; }

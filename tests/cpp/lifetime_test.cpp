@@ -16,6 +16,9 @@
 //                          tensors and models on the same context, as a
 //                          garbage collector's finaliser thread does; a
 //                          watchdog fails the run if the two deadlock
+//   lifetime_test config   gh_model_create's checks
+//   lifetime_test oom      a prefill whose longest pass does not fit in the
+//                          device memory takes shorter ones
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -25,6 +28,12 @@
 #include <vector>
 
 #include "gemma_hip.h"
+
+extern "C" size_t hip_stub_live_bytes(void);
+extern "C" void hip_stub_set_device_bytes(size_t n);
+namespace gh {
+extern std::vector<int> prefill_passes;
+}
 
 #define CHECK(c)                                                                                   \
     do {                                                                                           \
@@ -223,12 +232,66 @@ int config_checks() {
     return 0;
 }
 
+// A prefill takes the longest passes whose buffers fit: 2048, 1024 or 512
+// tokens; only what not even 512 fit in is GH_ERR_OOM.
+int prefill_oom() {
+    gh_ctx* ctx = nullptr;
+    gh_config c;
+    CHECK(gh_ctx_create(0, &ctx) == GH_OK);
+    CHECK(gh_config_preset("tiny", &c) == GH_OK);
+    const std::vector<int32_t> toks(1900, 3);
+    // bytes of the buffers for passes of n tokens; a prefill of 1900 tokens with `room` beside the model
+    auto run = [&](int n, size_t room, size_t* used, int* rc) {
+        gh_model* m = nullptr;
+        gh_kv* kv = nullptr;
+        CHECK(gh_model_create(ctx, &c, &m) == GH_OK);
+        CHECK(gh_synth_model(m, 7, 1, 0.02f, 0.01f, 0.02f) == GH_OK);
+        CHECK(gh_kv_create(m, 2048, &kv) == GH_OK);
+        int32_t next = -1;
+        CHECK(gh_step(m, kv, 3, nullptr, nullptr, &next) == GH_OK);
+        const size_t before = hip_stub_live_bytes();
+        gh::prefill_passes.clear();
+        hip_stub_set_device_bytes(room == SIZE_MAX ? room : before + room);
+        *rc = gh_prefill(m, kv, toks.data(), n, nullptr, nullptr, &next);
+        hip_stub_set_device_bytes(SIZE_MAX);
+        *used = hip_stub_live_bytes() - before;
+        if (*rc != GH_OK) {  // the failed call left nothing behind, and the next one works
+            int32_t len = -1;
+            CHECK(gh_kv_length(kv, &len) == GH_OK && len == 1 && *used == 0);
+            gh::prefill_passes.clear();
+            CHECK(gh_prefill(m, kv, toks.data(), n, nullptr, nullptr, &next) == GH_OK);
+        }
+        CHECK(gh_kv_destroy(kv) == GH_OK && gh_model_destroy(m) == GH_OK);
+        return 0;
+    };
+    const std::vector<int> one{1900}, two{1024, 876}, four{512, 512, 512, 364};
+    size_t used = 0, b512 = 0, b1024 = 0, b1920 = 0;
+    int rc = GH_OK;
+    if (run(512, SIZE_MAX, &b512, &rc) || run(1024, SIZE_MAX, &b1024, &rc) || run(1900, SIZE_MAX, &b1920, &rc)) return 1;
+    CHECK(b512 < b1024 && b1024 < b1920 && gh::prefill_passes == one);
+    if (run(1900, b1920, &used, &rc)) return 1;
+    CHECK(rc == GH_OK && used == b1920 && gh::prefill_passes == one);
+    if (run(1900, b1920 - 1, &used, &rc)) return 1;
+    CHECK(rc == GH_OK && used == b1024 && gh::prefill_passes == two);
+    if (run(1900, b1024 - 1, &used, &rc)) return 1;
+    CHECK(rc == GH_OK && used == b512 && gh::prefill_passes == four);
+    if (run(1900, b512 - 1, &used, &rc)) return 1;
+    CHECK(rc == GH_ERR_OOM && gh::prefill_passes == one);
+    CHECK(gh_ctx_destroy(ctx) == GH_OK);
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "config") == 0) {
         if (config_checks()) return 1;
         std::printf("config ok\n");
+        return 0;
+    }
+    if (argc > 1 && std::strcmp(argv[1], "oom") == 0) {
+        if (prefill_oom()) return 1;
+        std::printf("oom ok\n");
         return 0;
     }
     if (argc > 1 && std::strcmp(argv[1], "race") == 0) {

@@ -96,3 +96,11 @@ def test_model_create_rejects_unsupported_configs(lifetime_exe):
     capacity); hidden 3072 is accepted."""
     r = _run(lifetime_exe, "config")
     assert r.returncode == 0 and "config ok" in r.stdout, r.stdout + r.stderr[-4000:]
+
+
+def test_prefill_takes_shorter_passes_when_memory_is_short(lifetime_exe):
+    """1900 tokens with room for the buffers of one pass of 1920 rows, of
+    1024, of 512 and of none: one, two and four passes, and GH_ERR_OOM with
+    the cache unchanged and nothing held."""
+    r = _run(lifetime_exe, "oom")
+    assert r.returncode == 0 and "oom ok" in r.stdout, r.stdout + r.stderr[-4000:]
