@@ -19,6 +19,10 @@
 //   lifetime_test config   gh_model_create's checks
 //   lifetime_test oom      a prefill whose longest pass does not fit in the
 //                          device memory takes shorter ones
+//   lifetime_test cut FMT HIDDEN FFN N ...
+//                          per N: token tile, splits, blocks per split and
+//                          blocks of the four GEMMs of a prefill of N tokens
+//                          (8 q heads, 4 kv heads, head_dim 256)
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -27,7 +31,7 @@
 #include <thread>
 #include <vector>
 
-#include "gemma_hip.h"
+#include "../../gemma.hs_amd/csrc/common.h"
 
 extern "C" size_t hip_stub_live_bytes(void);
 extern "C" void hip_stub_set_device_bytes(size_t n);
@@ -281,6 +285,39 @@ int prefill_oom() {
     return 0;
 }
 
+int print_cuts(int argc, char** argv) {
+    CHECK(argc > 5);
+    const int fmt = std::atoi(argv[2]);
+    gh_ctx* ctx = nullptr;
+    gh_config c;
+    gh_model* m = nullptr;
+    CHECK(gh_ctx_create(0, &ctx) == GH_OK);
+    CHECK(gh_config_preset("gemma3-4b", &c) == GH_OK);
+    c.hidden = std::atoi(argv[3]);
+    c.ffn = std::atoi(argv[4]);
+    c.n_layers = 1;
+    CHECK(gh_model_create(ctx, &c, &m) == GH_OK);
+    auto set = [&](const char* name, size_t rows, size_t cols) {
+        const std::vector<uint8_t> zeros(fmt == gh::FMT_Q4 ? rows * (cols / 32) * 18 : rows * cols * 4);
+        return gh_model_set_tensor(m, name, fmt == gh::FMT_Q4 ? GH_DTYPE_Q4_0 : GH_DTYPE_F32, zeros.data(), zeros.size());
+    };
+    const size_t H = c.hidden, F = c.ffn, Q = (size_t)c.n_heads * c.head_dim;
+    CHECK(set("blk.0.attn_q.weight", Q, H) == GH_OK && set("blk.0.attn_output.weight", H, Q) == GH_OK);
+    CHECK(set("blk.0.ffn_gate.weight", F, H) == GH_OK && set("blk.0.ffn_down.weight", H, F) == GH_OK);
+    const gh::LayerDev& L = m->layers[0];
+    for (int i = 5; i < argc; ++i) {
+        const int n = std::atoi(argv[i]);
+        std::printf("%d", n);
+        for (const gh::DMat* w : {&L.qkv, &L.o, &L.gu, &L.down}) {
+            const gh::PfCut k = gh::pf_cut(*w, gh::pf_rows_padded(w->fmt, n));
+            std::printf(" %d,%d,%d,%d,%d", k.mt, k.S, k.per, w->nblk, w->cols);
+        }
+        std::printf("\n");
+    }
+    CHECK(gh_model_destroy(m) == GH_OK && gh_ctx_destroy(ctx) == GH_OK);
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -289,6 +326,7 @@ int main(int argc, char** argv) {
         std::printf("config ok\n");
         return 0;
     }
+    if (argc > 1 && std::strcmp(argv[1], "cut") == 0) return print_cuts(argc, argv);
     if (argc > 1 && std::strcmp(argv[1], "oom") == 0) {
         if (prefill_oom()) return 1;
         std::printf("oom ok\n");

@@ -17,6 +17,7 @@ import numpy as np
 import pytest
 
 import gemma_hip as gh
+import prefill_shapes
 import pyoracle as orc
 from conftest import GOLDEN, rel_err
 
@@ -122,10 +123,10 @@ def test_prefill_gqa_long_window_chunks_live_oracle(ctx):
 
 
 def test_prefill_passes_chunks_and_ragged_sizes(ctx):
-    """f32 tiny model, 600 tokens: one prefill call (two passes of 512 + 88
-    rows), the same tokens as prefills of 1, 63, 65, 7 and 464 tokens, and
-    the decode step token by token all reach the same last-token logits and
-    next token; the caches then continue identically."""
+    """f32 tiny model, 600 tokens: one prefill call (one pass), the same
+    tokens as prefills of 1, 63, 65, 7 and 464 tokens, and the decode step
+    token by token all reach the same last-token logits and next token; the
+    caches then continue identically."""
     cfg = gh.preset("tiny")
     m = _gpu_model(ctx, cfg, 7, False)
     toks = gh.synth_tokens(11, "long", 600, cfg.vocab)
@@ -164,6 +165,44 @@ def test_prefill_longer_than_a_pass(ctx):
     assert rel_err(la, lb) < ACT_TOL and na == nb
 
 
+def test_prefill_longer_than_a_pass_q4(ctx):
+    """The same pass boundary with Q4_0 weights and head_dim 256 (matrix-core
+    attention, shared key chunks, 128-row GEMM tiles) and a 300-position
+    window in the local layer: 2100 tokens as 2048 + 52 against 1000 + 1100."""
+    cfg = _mini4b(gh.MODE_GEMMA3, window=300, layers=2)
+    cfg.max_seq = 2304
+    m = _gpu_model(ctx, cfg, 43, True)
+    toks = gh.synth_tokens(17, "passq4", 2100, cfg.vocab)
+    kv_a, kv_b = gh.KVCache(m, 2304), gh.KVCache(m, 2304)
+    la, ya, na = gh.prefill(m, kv_a, toks, want_layers=True)
+    gh.prefill(m, kv_b, toks[:1000])
+    lb, yb, nb = gh.prefill(m, kv_b, toks[1000:], want_layers=True)
+    for l in range(cfg.n_layers):
+        assert rel_err(ya[l], yb[l]) < ACT_TOL, l
+    assert rel_err(la, lb) < ACT_TOL and na == nb
+
+
+@pytest.mark.parametrize("nq,nkv", [(4, 1), (8, 4)])
+@pytest.mark.parametrize("n", [1010, 1900])
+def test_prefill_attention_all_chunk_slots(ctx, nq, nkv, n):
+    """All 16 chunk states of the matrix-core attention and its merge (1010
+    tokens: 16 chunks of 64 positions; 1900: 15 of 128), in a global layer
+    and in one with a 200-position window: every layer of the last token
+    against the decode step fed token by token, ACT_TOL as above."""
+    cfg = _mini4b(gh.MODE_GEMMA3, window=200, layers=2)
+    cfg.n_heads, cfg.n_kv_heads, cfg.max_seq = nq, nkv, 1920
+    m = _gpu_model(ctx, cfg, 47, True)
+    toks = gh.synth_tokens(18, "slots", n, cfg.vocab)
+    kv_a, kv_b = gh.KVCache(m, 1920), gh.KVCache(m, 1920)
+    la, ya, na = gh.prefill(m, kv_a, toks, want_layers=True)
+    for t in toks[:-1]:
+        gh.runGemmaInferenceCached(m, int(t), kv_b, want_logits=False)
+    lb, _, yb, nb = gh.runGemmaInferenceCachedWithLayer0(m, int(toks[-1]), kv_b)
+    for l in range(cfg.n_layers):
+        assert rel_err(ya[l], yb[l]) < ACT_TOL, l
+    assert rel_err(la, lb) < ACT_TOL and na == nb
+
+
 @pytest.mark.parametrize("nq,nkv", [(4, 4), (8, 1)])
 def test_prefill_matrix_core_attention_groups_ragged_windows(ctx, nq, nkv):
     """head_dim 256 with GQA groups 1 and 8 (the 2 and 4 of the other tests
@@ -188,19 +227,20 @@ def test_prefill_matrix_core_attention_groups_ragged_windows(ctx, nq, nkv):
     np.testing.assert_array_equal(gh.generate(m, kv_a, [na], 5), gh.generate(m, kv_b, [nb], 5))
 
 
-@pytest.mark.parametrize("n", [2, 15, 16, 17, 32, 33, 64, 65, 128, 129, 257])
-def test_prefill_gemm_tile_edges(ctx, n):
-    """Q4_0 prefill GEMM at the edges of its token tiles (16, 32, 64, 128
-    rows), with odd column block counts (hidden 288: 9 blocks, ffn 352: 11)
-    and a ragged last weight tile: the last token's layers and logits against
-    the decode step fed token by token (other kernels, other sums; both are
-    within ACT_TOL / 2 of the oracle elsewhere, so ACT_TOL bounds their
-    difference)."""
+@pytest.mark.parametrize("hidden,ffn,n", prefill_shapes.cases(prefill_shapes.Q4_0))
+def test_prefill_gemm_tile_edges(ctx, hidden, ffn, n):
+    """Q4_0 prefill GEMM in every one of its token tiles (16, 32, 64, 128
+    rows) and around their edges, with one and several column splits, odd
+    column block counts (hidden 288 and 1056: 9 and 33 blocks, ffn 352 and
+    6944: 11 and 217) and a ragged last weight tile: the last token's layers
+    and logits against the decode step fed token by token (other kernels,
+    other sums; both are within ACT_TOL / 2 of the oracle elsewhere, so
+    ACT_TOL bounds their difference)."""
     cfg = _mini4b(gh.MODE_GEMMA3, window=40, layers=2)
-    cfg.hidden, cfg.ffn, cfg.max_seq = 288, 352, 272
+    cfg.hidden, cfg.ffn, cfg.max_seq = hidden, ffn, 400
     m = _gpu_model(ctx, cfg, 31, True)
     toks = gh.synth_tokens(13, "tile", n, cfg.vocab)
-    kv_a, kv_b = gh.KVCache(m, 272), gh.KVCache(m, 272)
+    kv_a, kv_b = gh.KVCache(m, 400), gh.KVCache(m, 400)
     la, ya, na = gh.prefill(m, kv_a, toks, want_layers=True)
     for t in toks[:-1]:
         gh.runGemmaInferenceCached(m, int(t), kv_b, want_logits=False)
@@ -210,16 +250,17 @@ def test_prefill_gemm_tile_edges(ctx, n):
     assert rel_err(la, lb) < ACT_TOL and na == nb
 
 
-@pytest.mark.parametrize("n", [2, 16, 17, 33, 64, 65, 130])
-def test_prefill_f32_gemm_tile_edges(ctx, n):
-    """f32 prefill GEMM at the edges of its token tiles (16, 32, 64 rows)
-    and of its rounds of column steps (hidden 288: 18 steps, ffn 352: 22):
-    as the Q4_0 test above, with its bound."""
+@pytest.mark.parametrize("hidden,ffn,n", prefill_shapes.cases(prefill_shapes.F32))
+def test_prefill_f32_gemm_tile_edges(ctx, hidden, ffn, n):
+    """f32 prefill GEMM in every one of its token tiles (16, 32, 64 rows),
+    below and above 512 columns, and around the edges of its rounds of column
+    steps (hidden 288: 18 steps, ffn 352: 22): as the Q4_0 test above, with
+    its bound."""
     cfg = _mini4b(gh.MODE_GEMMA3, window=40, layers=2)
-    cfg.hidden, cfg.ffn, cfg.max_seq = 288, 352, 144
+    cfg.hidden, cfg.ffn, cfg.max_seq = hidden, ffn, 272
     m = _gpu_model(ctx, cfg, 37, False)
     toks = gh.synth_tokens(15, "f32tile", n, cfg.vocab)
-    kv_a, kv_b = gh.KVCache(m, 144), gh.KVCache(m, 144)
+    kv_a, kv_b = gh.KVCache(m, 272), gh.KVCache(m, 272)
     la, ya, na = gh.prefill(m, kv_a, toks, want_layers=True)
     for t in toks[:-1]:
         gh.runGemmaInferenceCached(m, int(t), kv_b, want_logits=False)
@@ -336,10 +377,9 @@ def test_prefill_f32_sums_restart(ctx, ffn, n):
 @pytest.mark.parametrize("n", [16, 97, 300])
 def test_prefill_attention_chunks_outside_the_window(ctx, nq, nkv, n):
     """Chunk states of the matrix-core attention and their merge, per GQA
-    group, at one chunk, at shared chunks of 16 positions and past 16 of them
-    (300 tokens: 32-position chunks, most outside a 20-position window):
-    every layer of the last token against the decode step, ACT_TOL as
-    above."""
+    group, at one chunk, at shared chunks of 16 positions and of 32 or 48
+    (300 tokens: 10 or 7 chunks, most outside a 20-position window): every
+    layer of the last token against the decode step, ACT_TOL as above."""
     cfg = _mini4b(gh.MODE_GEMMA3, window=20, layers=2)
     cfg.n_heads, cfg.n_kv_heads, cfg.max_seq = nq, nkv, 304
     m = _gpu_model(ctx, cfg, 41, True)

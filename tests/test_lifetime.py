@@ -20,6 +20,7 @@ import subprocess
 
 import pytest
 
+import prefill_shapes
 from conftest import REPO
 
 CSRC = REPO / "gemma.hs_amd" / "csrc"
@@ -104,3 +105,23 @@ def test_prefill_takes_shorter_passes_when_memory_is_short(lifetime_exe):
     the cache unchanged and nothing held."""
     r = _run(lifetime_exe, "oom")
     assert r.returncode == 0 and "oom ok" in r.stdout, r.stdout + r.stderr[-4000:]
+
+
+@pytest.mark.parametrize("fmt,shapes", [(0, prefill_shapes.Q4_0), (1, prefill_shapes.F32)])
+def test_prefill_gemm_shapes_take_every_instance(lifetime_exe, fmt, shapes):
+    """The GPU tests' shapes launch every prefill GEMM instance: Q4_0 token
+    tiles of 16, 32, 64 and 128 rows, each with one and with several column
+    splits, and a last split of an odd number of blocks (tiles of 128 among
+    them); f32 tiles of 16, 32 and 64 rows on either side of 512 columns."""
+    seen, odd = set(), set()
+    for (hidden, ffn), ns in shapes.items():
+        r = _run(lifetime_exe, "cut", str(fmt), str(hidden), str(ffn), *map(str, ns))
+        assert r.returncode == 0, r.stdout + r.stderr[-4000:]
+        for line in r.stdout.splitlines():
+            for mt, splits, per, nblk, cols in (map(int, f.split(",")) for f in line.split()[1:]):
+                assert (splits - 1) * per < nblk <= splits * per
+                seen.add((mt, splits > 1) if fmt == 0 else (mt, cols < 512))
+                if splits > 1 and (nblk - (splits - 1) * per) % 2:
+                    odd.add(mt)
+    assert seen == {(mt, b) for mt in ((16, 32, 64, 128) if fmt == 0 else (16, 32, 64)) for b in (False, True)}
+    assert fmt == 1 or odd >= {16, 32, 64, 128}
