@@ -189,6 +189,7 @@ struct Sink {
 // Buffers of the batched prompt prefill (per model, grown on demand).
 struct PfBufs {
     int cap = 0;                 // token rows (multiple of 128) the row buffers hold
+    void* block = nullptr;       // the one allocation that holds them all
     float* x = nullptr;          // [cap][H] residual after attention / after the layer
     float* x1 = nullptr;         // [cap][H] residual after attention
     void* a = nullptr;           // [2][cap][Kmax] fp16 (Q4_0 weights) or [cap][Kmax] f32: GEMM operand

@@ -31,7 +31,7 @@ std::map<void*, size_t>& live_allocs() {
     static auto* s = new std::map<void*, size_t>();
     return *s;
 }
-size_t live_bytes = 0, device_bytes = SIZE_MAX;
+size_t live_bytes = 0, device_bytes = SIZE_MAX, mallocs = 0;
 
 // Reads the object's first word: a use-after-free under AddressSanitizer.
 hipError_t touch(const void* o, unsigned magic) {
@@ -48,6 +48,7 @@ hipError_t dev_alloc(void** p, size_t n) {
     *p = std::malloc(n ? n : 1);
     live_allocs()[*p] = n;
     live_bytes += n;
+    mallocs += 1;
     return hipSuccess;
 }
 
@@ -75,6 +76,10 @@ extern "C" {
 size_t hip_stub_live_bytes(void) {
     std::lock_guard<std::mutex> g(mu());
     return live_bytes;
+}
+size_t hip_stub_mallocs(void) {
+    std::lock_guard<std::mutex> g(mu());
+    return mallocs;
 }
 void hip_stub_set_device_bytes(size_t n) {
     std::lock_guard<std::mutex> g(mu());

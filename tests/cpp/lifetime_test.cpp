@@ -34,6 +34,7 @@
 #include "../../gemma.hs_amd/csrc/common.h"
 
 extern "C" size_t hip_stub_live_bytes(void);
+extern "C" size_t hip_stub_mallocs(void);
 extern "C" void hip_stub_set_device_bytes(size_t n);
 namespace gh {
 extern std::vector<int> prefill_passes;
@@ -236,8 +237,8 @@ int config_checks() {
     return 0;
 }
 
-// A prefill takes the longest passes whose buffers fit: 2048, 1024 or 512
-// tokens; only what not even 512 fit in is GH_ERR_OOM.
+// A prefill takes the longest passes whose buffers fit: the whole prompt (to
+// 2048 tokens), 1024 or 512; only what not even 512 fit in is GH_ERR_OOM.
 int prefill_oom() {
     gh_ctx* ctx = nullptr;
     gh_config c;
@@ -269,18 +270,37 @@ int prefill_oom() {
         return 0;
     };
     const std::vector<int> one{1900}, two{1024, 876}, four{512, 512, 512, 364};
-    size_t used = 0, b512 = 0, b1024 = 0, b1920 = 0;
+    size_t used = 0, b512 = 0, b1024 = 0, b2048 = 0;
     int rc = GH_OK;
-    if (run(512, SIZE_MAX, &b512, &rc) || run(1024, SIZE_MAX, &b1024, &rc) || run(1900, SIZE_MAX, &b1920, &rc)) return 1;
-    CHECK(b512 < b1024 && b1024 < b1920 && gh::prefill_passes == one);
-    if (run(1900, b1920, &used, &rc)) return 1;
-    CHECK(rc == GH_OK && used == b1920 && gh::prefill_passes == one);
-    if (run(1900, b1920 - 1, &used, &rc)) return 1;
+    if (run(512, SIZE_MAX, &b512, &rc) || run(1024, SIZE_MAX, &b1024, &rc) || run(1900, SIZE_MAX, &b2048, &rc)) return 1;
+    CHECK(b512 < b1024 && b1024 < b2048 && gh::prefill_passes == one);
+    if (run(1900, b2048, &used, &rc)) return 1;
+    CHECK(rc == GH_OK && used == b2048 && gh::prefill_passes == one);
+    if (run(1900, b2048 - 1, &used, &rc)) return 1;
+    CHECK(rc == GH_OK && used < b2048 && used > b1024 && gh::prefill_passes == one);
+    if (run(1900, b1024, &used, &rc)) return 1;
     CHECK(rc == GH_OK && used == b1024 && gh::prefill_passes == two);
     if (run(1900, b1024 - 1, &used, &rc)) return 1;
     CHECK(rc == GH_OK && used == b512 && gh::prefill_passes == four);
     if (run(1900, b512 - 1, &used, &rc)) return 1;
     CHECK(rc == GH_ERR_OOM && gh::prefill_passes == one);
+    if (run(300, b512 - 1, &used, &rc)) return 1;
+    CHECK(rc == GH_OK && used < b512);
+    // prompts each longer than the one before: the buffers double, in one block
+    gh_model* m = nullptr;
+    gh_kv* kv = nullptr;
+    CHECK(gh_model_create(ctx, &c, &m) == GH_OK);
+    CHECK(gh_synth_model(m, 7, 1, 0.02f, 0.01f, 0.02f) == GH_OK);
+    CHECK(gh_kv_create(m, 2048, &kv) == GH_OK);
+    int32_t next = -1;
+    CHECK(gh_step(m, kv, 3, nullptr, nullptr, &next) == GH_OK);
+    const size_t mallocs = hip_stub_mallocs();
+    for (int n = 2; n <= 1900; n += 26) {
+        CHECK(gh_kv_truncate(kv, 0) == GH_OK);
+        CHECK(gh_prefill(m, kv, toks.data(), n, nullptr, nullptr, &next) == GH_OK);
+    }
+    CHECK(hip_stub_mallocs() - mallocs <= 5);
+    CHECK(gh_kv_destroy(kv) == GH_OK && gh_model_destroy(m) == GH_OK);
     CHECK(gh_ctx_destroy(ctx) == GH_OK);
     return 0;
 }

@@ -100,9 +100,10 @@ def test_model_create_rejects_unsupported_configs(lifetime_exe):
 
 
 def test_prefill_takes_shorter_passes_when_memory_is_short(lifetime_exe):
-    """1900 tokens with room for the buffers of one pass of 1920 rows, of
-    1024, of 512 and of none: one, two and four passes, and GH_ERR_OOM with
-    the cache unchanged and nothing held."""
+    """1900 tokens with room for the buffers of one pass, of 1024 rows, of 512
+    and of none: one, two and four passes, and GH_ERR_OOM with the cache
+    unchanged and nothing held.  Prompts each longer than the one before
+    allocate at most 5 times."""
     r = _run(lifetime_exe, "oom")
     assert r.returncode == 0 and "oom ok" in r.stdout, r.stdout + r.stderr[-4000:]
 
