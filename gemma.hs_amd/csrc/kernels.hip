@@ -4197,7 +4197,6 @@ int enqueue_step(gh_model* m, gh_kv* kv, Sink& sink, int pos) {
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 // GEMM operand A, [Pp][K] per part.
 // With Q4_0 weights (split = 1), each token row t is first scaled by a power
@@ -4365,12 +4364,12 @@ struct PfGemm {
     int kb_per;  // column blocks per split
     float* out;  // [S][Pp][ldo]
     int ldo;
-    int X, Y, S;  // row groups, 64-token tiles, splits (the grid is 1-D, see pf_tile)
+    int X, Y, S;  // weight tiles, token tiles of PfCut::mt rows, splits (the grid is 1-D, see pf_tile)
 };
 
 // XCD-aware workgroup order of the 1-D prefill GEMM grid.  Workgroups go to
 // the 8 XCDs round-robin (XCD = id % 8), each XCD with its own L2.  Key =
-// (row group x, split z) names the weight slice a workgroup reads; key k
+// (weight tile x, split z) names the weight slice a workgroup reads; key k
 // runs on XCD k % 8, and its Y token tiles run back to back there, so the
 // slice is fetched from HBM once.  With 8 splits, split z lives on XCD z
 // only, so its column slice of A is fetched by one L2 as well.  Ids past
@@ -4435,14 +4434,14 @@ __device__ __forceinline__ f16x8_t q4_f16x8(uint32_t w0, uint32_t w1, uint32_t b
 //     11.46 ms); runs of 16 would leave o_proj's sum of 32 blocks longer than
 //     its 4 splits of 8 once were.  Unrolling the run to put its adds between
 //     the MFMAs spills (91 VGPRs).
-// The 128 x 128 tile takes 0.55 us per block and CU, whether one or two
-// workgroups share the CU: per wave 32 MFMAs (512 cycles), 95 VALU
-// instructions (64 of them the scale FMAs) and 20 LDS ones.  Four blocks in
-// flight instead of two, stages of two or four blocks per barrier and
-// v_mfma_f32_32x32x16_f16 measured the same.  Against the 64 x 128 tile it
-// replaced (16 tokens a wave, whose LDS reads took as long as its MFMAs), 512
-// tokens: 1B gate/up 49 -> 43 us, 4B gate/up 135 -> 122, qkv 45 -> 30, down
-// 79 -> 66.
+// The 128 x 128 tile takes 0.57 us per block and CU with two workgroups on it
+// (0.55 without the restarts), 0.69 with one, launch included: per wave 32
+// MFMAs (512 cycles), 110 VALU instructions (64 of them the scale FMAs, 16
+// the restarts) and 21 LDS ones.  Four blocks in flight instead of two, stages of
+// two or four blocks per barrier and v_mfma_f32_32x32x16_f16 measured the
+// same.  Against the 64 x 128 tile it replaced (16 tokens a wave, whose LDS
+// reads took as long as its MFMAs), 512 tokens: 1B gate/up 49 -> 42 us, 4B
+// gate/up 135 -> 131, qkv 45 -> 31, down 79 -> 71.
 constexpr int PF_RUN = 8;  // column blocks a sum runs over (even)
 template <int MW, int TM, int TN>
 __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
@@ -4626,7 +4625,7 @@ __global__ __launch_bounds__(NT, 2) void k_pf_gemm_q4(PfGemm g) {
 // ahead, with no LDS and no barrier.  Each RUN steps are summed from zero and
 // then added to the running sum, which keeps the rounding error below that of
 // one chain over all the columns.  1B shape, 300 tokens: gate/up
-// 709 -> 117 us (82 TFLOP/s; the f32 matrix peak this card reaches is 138), down
+// 709 -> 117 us (82 TFLOP/s; a large f32 product reaches 152 on this card), down
 // 424 -> 72; the kernel before it waited on one load per MFMA.
 template <int TM, int RUN>
 __global__ __launch_bounds__(NT, 2) void k_pf_gemm_f32(PfGemm g) {

@@ -26,9 +26,16 @@ int pf_rows_padded(int fmt, int n) {
 // with what MI355X measured for one workgroup on a CU: 0.28 / 0.30 / 0.38 /
 // 0.55 us per 32-column Q4_0 block at 16 / 32 / 64 / 128 token rows, 0.21 /
 // 0.33 / 0.55 us per 16-column f32 step at 16 / 32 / 64, and 0.58 us per MB of
-// partials.  Over sweeps of S at 16 .. 1907 tokens of the 1B and 4B shapes it
-// picks the best S or one whose GEMM plus consumer is within 3 us of it, but
-// for 1024-token 1B down (3 splits, 62 us with its consumer; 6 take 55).
+// partials.  Against every tile and S, by the time of a whole layer (1B 7 to
+// 1907 tokens, 4B 16 to 1024, 1B f32 16 to 512; 96 matrices): 85 choices are
+// the best or within 3 us of it.  The other 11 lose 3.4 to 13 us, 1 to 4 % of
+// the layer, most of them by too few splits (4B 1024 tokens o_proj 44 us in
+// one split of 128-row tiles, 33 in two of 64; 4B 257 down 53 in 4, 44 in 8;
+// 4B 512 gate/up 131 in one, 116 in two; 1B 1907 qkv 29 in one, 24 in two).
+// Two things that the estimate leaves out: a workgroup alone on its CU takes
+// longer a block than one of two that share it take together (128 rows 0.69
+// us, launch included, against 0.57), and a key's token tiles stay on one XCD
+// (pf_tile), so the fullest XCD makes the round.
 PfCut pf_cut(const DMat& w, int Pp) {
     static const double q4_us[] = {0.28, 0.30, 0.38, 0.55}, f32_us[] = {0.21 / 4, 0.33 / 4, 0.55 / 4};  // per block
     const bool q4 = w.fmt == FMT_Q4;
