@@ -4436,7 +4436,7 @@ __device__ __forceinline__ f16x8_t q4_f16x8(uint32_t w0, uint32_t w1, uint32_t b
 //     the MFMAs spills (91 VGPRs).
 // The 128 x 128 tile takes 0.57 us per block and CU with two workgroups on it
 // (0.55 without the restarts), 0.69 with one, launch included: per wave 32
-// MFMAs (512 cycles), 110 VALU instructions (64 of them the scale FMAs, 16
+// MFMAs (512 cycles), 100 VALU instructions (64 of them the scale FMAs, 16
 // the restarts) and 21 LDS ones.  Four blocks in flight instead of two, stages of
 // two or four blocks per barrier and v_mfma_f32_32x32x16_f16 measured the
 // same.  Against the 64 x 128 tile it replaced (16 tokens a wave, whose LDS
